@@ -129,6 +129,12 @@ __global__ void k_cc_final(uint32_t n, uint32_t *p, uint32_t *out) {
   out[v] = cc::find(p, (uint32_t)v);
 }
 
+__global__ void k_cc_labels(cc::Slots sl, uint32_t *p, const uint32_t *low,
+                            uint32_t *out) {
+  const uint64_t v = (uint64_t)blockIdx.x * kT + threadIdx.x;
+  if (v < sl.n) out[v] = cc::label_of(sl, (uint32_t)v, p, low);
+}
+
 // ------------------------------------------------------------------ TC
 // lower[v] = number of neighbours of v below v.
 __global__ void k_lower_degree(DevGraph g, uint32_t *lower) {
@@ -941,20 +947,20 @@ int algo_cc(sstg_graph *g, uint32_t *out) {
   SSTG_TRY(graph_is_symmetric(g, &symmetric));
   const DevGraph v = g->view();
   if (g->m && symmetric) {
-    SSTG_LAUNCH(cc::k_identity, blocks(n), kT, 0, s, n, p);
-    SSTG_LAUNCH(cc::k_link_sample, blocks(n), kT, 0, s, v, p);
-    SSTG_LAUNCH(cc::k_compress, blocks(n), kT, 0, s, n, p);
-    SSTG_LAUNCH(cc::k_mode, 1, kT, 0, s, (const uint32_t *)nullptr, 1u, n, p,
-                giant);
-    SSTG_LAUNCH(cc::k_link_rest, blocks(n), kT, 0, s, v, p,
-                (const uint32_t *)giant, (const uint32_t *)nullptr);
+    uint32_t *samples = nullptr;
+    // PageRank's contribution buffer holds the same bytes (8 per vertex)
+  SSTG_TRY(g->ws.get(kWsAlgo + 20, (uint64_t)n * cc::kHookRounds, &samples));
+    const cc::Slots sl{prefix, nullptr, nullptr, n};
+    SSTG_TRY(cc::forest_symmetric(v, sl, p, samples, 1, giant, s));
+    SSTG_LAUNCH(k_cc_labels, blocks(n), kT, 0, s, sl, p,
+                (const uint32_t *)samples, out);
   } else {
     SSTG_LAUNCH(cc::k_init, blocks(n), kT, 0, s, v, p);
     if (g->m)
       SSTG_LAUNCH(cc::k_hook_all, ceil_div(ceil_div(g->m, 8), kT), kT, 0, s, v,
                 prefix, g->m, p);
+    SSTG_LAUNCH(k_cc_final, blocks(n), kT, 0, s, n, p, out);
   }
-  SSTG_LAUNCH(k_cc_final, blocks(n), kT, 0, s, n, p, out);
   SSTG_HIP(hipStreamSynchronize(s));
   return SSTG_OK;
 }

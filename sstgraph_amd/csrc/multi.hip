@@ -155,6 +155,13 @@ __global__ void k_mcc_final(uint32_t n, const uint32_t *vbase,
   label[v] = cc::find(p, (uint32_t)v) - vbase[graph_of[v]];
 }
 
+__global__ void k_mcc_labels(cc::Slots sl, uint32_t *p, const uint32_t *low,
+                             uint32_t *label) {
+  const uint64_t v = (uint64_t)blockIdx.x * kT + threadIdx.x;
+  if (v < sl.n)
+    label[v] = cc::label_of(sl, (uint32_t)v, p, low) - sl.vbase[sl.graph_of[v]];
+}
+
 // ---- PageRank over the union with per-graph normalisation
 template <class Real>
 __global__ void k_mpr_init(uint32_t n, const uint32_t *deg,
@@ -289,6 +296,9 @@ static int capture(sstg_multi *M, uint32_t max_levels, uint32_t iters,
   SSTG_TRY(degree_bins(g, &bins, kBinsPull));
   bool symmetric = false;
   SSTG_TRY(graph_is_symmetric(g, &symmetric));
+  uint32_t *samples = nullptr;
+  // PageRank's contribution buffer holds the same bytes (8 per vertex)
+  SSTG_TRY(g->ws.get(kWsAlgo + 20, (uint64_t)n * cc::kHookRounds, &samples));
   SSTG_HIP(hipStreamSynchronize(s));
   // the event profiler must not record into a capturing stream
   Profiler &prof = profiler();
@@ -314,19 +324,11 @@ static int capture(sstg_multi *M, uint32_t max_levels, uint32_t iters,
     // CC
     const DevGraph v = g->view();
     if (g->m && symmetric) {
-      hipLaunchKernelGGL(cc::k_identity, dim3(blocks(n)), dim3(kT), 0, s, n,
-                         M->uf);
-      hipLaunchKernelGGL(cc::k_link_sample, dim3(blocks(n)), dim3(kT), 0, s, v,
-                         M->uf);
-      hipLaunchKernelGGL(cc::k_compress, dim3(blocks(n)), dim3(kT), 0, s, n,
-                         M->uf);
-      hipLaunchKernelGGL(cc::k_mode,
-                         dim3(ceil_div((uint64_t)M->k * kWave, kT)), dim3(kT),
-                         0, s, (const uint32_t *)M->d_vbase, M->k, n, M->uf,
-                         M->giant);
-      hipLaunchKernelGGL(cc::k_link_rest, dim3(blocks(n)), dim3(kT), 0, s, v,
-                         M->uf, (const uint32_t *)M->giant,
-                         (const uint32_t *)M->d_graph_of);
+      const cc::Slots sl{prefix, M->d_vbase, M->d_graph_of, n};
+      rc = cc::forest_symmetric(v, sl, M->uf, samples, M->k, M->giant, s);
+      if (rc != SSTG_OK) break;
+      hipLaunchKernelGGL(k_mcc_labels, dim3(blocks(n)), dim3(kT), 0, s, sl,
+                         M->uf, (const uint32_t *)samples, M->label);
     } else {
       hipLaunchKernelGGL(cc::k_init, dim3(blocks(n)), dim3(kT), 0, s, v,
                          M->uf);
@@ -334,10 +336,10 @@ static int capture(sstg_multi *M, uint32_t max_levels, uint32_t iters,
         hipLaunchKernelGGL(cc::k_hook_all,
                            dim3(ceil_div(ceil_div(g->m, 8), kT)), dim3(kT), 0,
                            s, v, prefix, g->m, M->uf);
+      hipLaunchKernelGGL(k_mcc_final, dim3(blocks(n)), dim3(kT), 0, s, n,
+                         (const uint32_t *)M->d_vbase,
+                         (const uint32_t *)M->d_graph_of, M->uf, M->label);
     }
-    hipLaunchKernelGGL(k_mcc_final, dim3(blocks(n)), dim3(kT), 0, s, n,
-                       (const uint32_t *)M->d_vbase,
-                       (const uint32_t *)M->d_graph_of, M->uf, M->label);
     // PageRank
     if (f32)
       rc = record_pagerank<float, true>(M, bins, iters, damping, M->rank32,
