@@ -636,26 +636,10 @@ struct DegreeBins {
   uint64_t count[4] = {0, 0, 0, 0};
 };
 
-namespace em {
-namespace {  // internal linkage: this header is included by several files
-__global__ void k_bin_flags(const uint32_t *deg, uint32_t n, uint32_t lo,
-                            uint32_t hi, uint8_t *flags) {
-  uint64_t v = (uint64_t)blockIdx.x * kT + threadIdx.x;
-  if (v < n) {
-    uint32_t d = deg[v];
-    flags[v] = d >= lo && d <= hi;
-  }
-}
-}  // namespace
-}  // namespace em
-
 // The four lists lie back to back in one buffer (list[b + 1] = list[b] +
 // count[b]).
 inline int degree_bins(sstg_graph *g, DegreeBins *out, int set = kBinsPull) {
   const uint32_t *t = g->bin_hi[set];
-  const uint32_t lo[4] = {0, t[0] + 1, t[1] + 1, t[2] + 1};
-  const uint32_t hi[4] = {t[0], t[1], t[2], 0xFFFFFFFFu};
-  hipStream_t s = g->stream;
   const uint32_t n = g->n_rows;
   const int slot = set == kBinsPull ? kWsAlgo + 26 : kWsBfsBins;
   uint32_t *all = nullptr;
@@ -669,22 +653,10 @@ inline int degree_bins(sstg_graph *g, DegreeBins *out, int set = kBinsPull) {
     }
     return SSTG_OK;
   }
-  uint8_t *flags = nullptr;
-  uint64_t *tmp = nullptr;
-  SSTG_TRY(g->ws.get(kWsAlgo + 24, n, &flags));
-  SSTG_TRY(g->ws.get(kWsAlgo + 25, n, &tmp));
-  for (int b = 0; b < 4; b++) {
-    SSTG_LAUNCH(em::k_bin_flags, ceil_div(n, em::kT), em::kT, 0, s,
-                (const uint32_t *)g->deg, n, lo[b], hi[b], flags);
-    SSTG_TRY(select_flagged_u64(flags, nullptr, n, tmp, g->dev_ctr + 7, g->ws,
-                                kWsPrim, s));
-    SSTG_HIP(hipMemcpyAsync(g->host_rb + 16, g->dev_ctr + 7, sizeof(uint64_t),
-                            hipMemcpyDeviceToHost, s));
-    SSTG_HIP(hipStreamSynchronize(s));
-    out->count[b] = g->host_rb[16];
-    out->list[b] = all + (b ? (out->list[b - 1] - all) + out->count[b - 1] : 0);
-    SSTG_TRY(narrow_u64_to_u32(tmp, out->count[b], out->list[b], s));
-  }
+  const uint32_t hi[4] = {t[0], t[1], t[2], 0xFFFFFFFFu};
+  SSTG_TRY(graph_bins(g, g->deg, 0, hi, 4, all, out->count, nullptr));
+  out->list[0] = all;
+  for (int b = 1; b < 4; b++) out->list[b] = out->list[b - 1] + out->count[b - 1];
   for (int b = 0; b < 4; b++) g->bins_count[set][b] = out->count[b];
   g->bins_version[set] = g->version;
   return SSTG_OK;

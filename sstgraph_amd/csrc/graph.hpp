@@ -114,8 +114,9 @@ int graph_alloc(sstg_graph *g);
 void graph_free(sstg_graph *g);
 // host_ctr holds kHostCtrSlots words: the counter blocks from 0 and, at
 // kHostFlag, the sequence number a kernel writes after them
-constexpr int kHostCtrSlots = 32;
+constexpr int kHostCtrSlots = 64;
 constexpr int kHostFlag = 24;
+constexpr int kHostBins = 32;  // graph_bins: the totals
 
 // Waits until the device has written seq to host_ctr[kHostFlag] (spinning on
 // the mapped word, which arrives as soon as the kernel writes it rather than
@@ -126,6 +127,14 @@ int wait_host_flag(sstg_graph *g, uint64_t seq);
 
 int graph_update(sstg_graph *g, const uint32_t *src, const uint32_t *dst,
                  uint64_t n, bool insert, bool skip_self, bool device_ptrs);
+// primitives.hip: the vertices split by val[v] into bins lists, ascending and
+// back to back in list (n_rows entries): bin 0 holds lo <= val <= hi[0], bin b
+// hi[b - 1] < val <= hi[b]; counts[b] gets their lengths, *largest the largest
+// value of all.  Waits for the counts (not for the lists).
+constexpr int kMaxBins = 6;
+int graph_bins(sstg_graph *g, const uint32_t *val, uint32_t lo,
+               const uint32_t *hi, int bins, uint32_t *list, uint64_t *counts,
+               uint64_t *largest);
 int graph_rebuild(sstg_graph *g, uint64_t extra_elems);
 int graph_effective_keys(sstg_graph *g, const uint32_t *src,
                          const uint32_t *dst, uint64_t n, bool insert,
@@ -234,6 +243,7 @@ enum : int {
   kWsSmallRows = 147,
   kWsSmallFound = 149,  // small updates: each pair's row search
   kWsRebuild = 150,     // 150..152 pool rebuild: capacities, offsets, prefix
+  kWsBins = 153,        // 153, 154 graph_bins: block counts, totals
 };
 
 // degree threshold sets of a graph (sstg_graph::bin_hi): the reductions

@@ -212,6 +212,189 @@ __global__ void __launch_bounds__(kScanThreads)
     *d_count = carry;
 }
 
+// ------------------------------------------------------------- bins
+// Vertices split by a value into up to kMaxBins lists, in order, in three
+// launches and one host wait whatever the number of bins: each block counts
+// its range per bin, one block scans the bins x blocks counts, and each block
+// writes its range to the lists.  A wave's place within a bin comes from a
+// ballot per bin, so a step of 1024 values costs two barriers.
+constexpr int kBinSteps = 4;  // values per thread and step
+constexpr uint64_t kBinStep = kScanThreads * kBinSteps;
+constexpr uint64_t kBinBlocks = 1024;
+constexpr int kBinScanThreads = 1024;
+
+struct BinSpec {
+  uint32_t lo, hi[kMaxBins];  // bin b: (hi[b - 1], hi[b]], bin 0 from lo
+  int bins;
+};
+
+__device__ __forceinline__ int bin_of(const BinSpec &sp, uint32_t v) {
+  if (v < sp.lo) return -1;
+  int b = 0;
+#pragma unroll
+  for (int k = 0; k + 1 < kMaxBins; k++)
+    if (k + 1 < sp.bins && v > sp.hi[k]) b = k + 1;
+  return b;
+}
+
+// cnt[b * blocks + block], and the block's largest value in
+// cnt[bins * blocks + block]
+__global__ void __launch_bounds__(kScanThreads)
+    k_bins_count(const uint32_t *val, uint64_t n, uint64_t per, BinSpec sp,
+                 uint32_t *cnt) {
+  __shared__ uint32_t wc[kScanThreads / kWave][kMaxBins + 1];
+  const uint64_t lo = (uint64_t)blockIdx.x * per;
+  const uint64_t hi = lo + per < n ? lo + per : n;
+  const int w = threadIdx.x / kWave;
+  uint32_t c[kMaxBins] = {}, top = 0;
+  for (uint64_t i0 = lo; i0 < hi; i0 += kBinStep) {
+    uint32_t v[kBinSteps];
+#pragma unroll
+    for (int j = 0; j < kBinSteps; j++) {
+      const uint64_t i = i0 + (uint64_t)j * kScanThreads + threadIdx.x;
+      v[j] = val[i < hi ? i : hi - 1];
+    }
+#pragma unroll
+    for (int j = 0; j < kBinSteps; j++) {
+      const uint64_t i = i0 + (uint64_t)j * kScanThreads + threadIdx.x;
+      const int b = i < hi ? bin_of(sp, v[j]) : -1;
+      top = v[j] > top ? v[j] : top;
+#pragma unroll
+      for (int k = 0; k < kMaxBins; k++)
+        c[k] += (uint32_t)__popcll(__ballot(b == k));
+    }
+  }
+#pragma unroll
+  for (int o = kWave / 2; o > 0; o >>= 1) {
+    const uint32_t t = __shfl_xor(top, o, kWave);
+    top = t > top ? t : top;
+  }
+  if ((threadIdx.x & (kWave - 1)) == 0) {
+#pragma unroll
+    for (int k = 0; k < kMaxBins; k++) wc[w][k] = c[k];
+    wc[w][kMaxBins] = top;
+  }
+  __syncthreads();
+  if (threadIdx.x <= (uint32_t)sp.bins) {
+    const bool is_top = threadIdx.x == (uint32_t)sp.bins;
+    uint32_t t = 0;
+    for (int i = 0; i < kScanThreads / kWave; i++) {
+      const uint32_t x = wc[i][is_top ? kMaxBins : threadIdx.x];
+      t = is_top ? (x > t ? x : t) : t + x;
+    }
+    cnt[(uint64_t)threadIdx.x * gridDim.x + blockIdx.x] = t;
+  }
+}
+
+// One block: the exclusive scan of the counts in place (bin-major, so a
+// bin's list starts where the one before ends); tot[b] = entries of bin b,
+// tot[bins] = the largest value, copied to the host's block with the flag
+// behind it when there is one.
+__global__ void __launch_bounds__(kBinScanThreads)
+    k_bins_scan(uint32_t *cnt, uint32_t blocks, int bins, uint64_t *tot,
+                uint64_t *host, uint64_t *host_flag, uint64_t seq) {
+  __shared__ uint32_t wtot[kBinScanThreads / kWave];
+  __shared__ uint32_t first[kMaxBins + 1], wtop[kBinScanThreads / kWave];
+  const uint32_t lane = lane_id(), w = threadIdx.x / kWave;
+  const uint32_t n = blocks * (uint32_t)bins;
+  uint32_t carry = 0;
+  for (uint32_t c0 = 0; c0 < n; c0 += kBinScanThreads) {  // uniform
+    const uint32_t i = c0 + threadIdx.x;
+    const uint32_t v = i < n ? cnt[i] : 0;
+    const uint32_t incl = wave_inclusive_sum(v);
+    if (lane == kWave - 1) wtot[w] = incl;
+    __syncthreads();
+    uint32_t off = carry, all = 0;
+    for (uint32_t k = 0; k < kBinScanThreads / kWave; k++) {
+      const uint32_t x = wtot[k];
+      if (k < w) off += x;
+      all += x;
+    }
+    __syncthreads();
+    if (i < n) {
+      cnt[i] = off + incl - v;
+      if (i % blocks == 0) first[i / blocks] = off + incl - v;
+    }
+    carry += all;
+  }
+  uint32_t top = 0;
+  for (uint32_t i = threadIdx.x; i < blocks; i += kBinScanThreads) {
+    const uint32_t x = cnt[n + i];
+    top = x > top ? x : top;
+  }
+#pragma unroll
+  for (int o = kWave / 2; o > 0; o >>= 1) {
+    const uint32_t t = __shfl_xor(top, o, kWave);
+    top = t > top ? t : top;
+  }
+  if (lane == 0) wtop[w] = top;
+  if (threadIdx.x == 0) first[bins] = carry;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (uint32_t k = 1; k < kBinScanThreads / kWave; k++)
+      top = wtop[k] > top ? wtop[k] : top;
+    for (int b = 0; b <= bins; b++) {
+      const uint64_t x = b < bins ? first[b + 1] - first[b] : top;
+      tot[b] = x;
+      if (host) host[b] = x;
+    }
+    if (host) {
+      __threadfence_system();  // the totals before the flag, to the host
+      *(volatile uint64_t *)host_flag = seq;
+    }
+  }
+}
+
+__global__ void __launch_bounds__(kScanThreads)
+    k_bins_place(const uint32_t *val, uint64_t n, uint64_t per, BinSpec sp,
+                 const uint32_t *cnt, uint32_t *list) {
+  __shared__ uint32_t wc[kScanThreads / kWave][kMaxBins];
+  __shared__ uint32_t at[kMaxBins];
+  const uint64_t lo = (uint64_t)blockIdx.x * per;
+  const uint64_t hi = lo + per < n ? lo + per : n;
+  const uint32_t w = threadIdx.x / kWave, lane = lane_id();
+  if (threadIdx.x < (uint32_t)sp.bins)
+    at[threadIdx.x] = cnt[(uint64_t)threadIdx.x * gridDim.x + blockIdx.x];
+  for (uint64_t i0 = lo; i0 < hi; i0 += kBinStep) {
+    // a wave's values are consecutive, so its entries are in order
+    const uint64_t wi = i0 + (uint64_t)w * kWave * kBinSteps + lane;
+    int b[kBinSteps];
+    uint32_t v[kBinSteps], rank[kBinSteps], c[kMaxBins] = {};
+#pragma unroll
+    for (int j = 0; j < kBinSteps; j++) {
+      const uint64_t i = wi + (uint64_t)j * kWave;
+      v[j] = val[i < hi ? i : hi - 1];
+    }
+#pragma unroll
+    for (int j = 0; j < kBinSteps; j++) {
+      b[j] = wi + (uint64_t)j * kWave < hi ? bin_of(sp, v[j]) : -1;
+      rank[j] = 0;
+#pragma unroll
+      for (int k = 0; k < kMaxBins; k++) {
+        const uint64_t m = __ballot(b[j] == k);
+        if (b[j] == k) rank[j] = c[k] + mask_rank(m);
+        c[k] += (uint32_t)__popcll(m);
+      }
+    }
+    if (lane == 0)
+#pragma unroll
+      for (int k = 0; k < kMaxBins; k++) wc[w][k] = c[k];
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < kBinSteps; j++)
+      if (b[j] >= 0) {
+        uint32_t o = at[b[j]] + rank[j];
+        for (uint32_t k = 0; k < w; k++) o += wc[k][b[j]];
+        list[o] = (uint32_t)(wi + (uint64_t)j * kWave);
+      }
+    __syncthreads();
+    if (threadIdx.x < (uint32_t)sp.bins)
+      for (uint32_t k = 0; k < kScanThreads / kWave; k++)
+        at[threadIdx.x] += wc[k][threadIdx.x];
+    __syncthreads();
+  }
+}
+
 // --------------------------------------------------------- radix sort
 constexpr int kRsThreads = 256;
 constexpr int kRsWaves = kRsThreads / kWave;
@@ -761,6 +944,46 @@ int select_flagged_u32(const uint8_t *flags, const uint32_t *values,
                        Workspace &ws, int ws_base, hipStream_t s) {
   return select_flagged<uint32_t>(flags, values, n, out, d_count, ws, ws_base,
                                   s);
+}
+
+int graph_bins(sstg_graph *g, const uint32_t *val, uint32_t lo,
+               const uint32_t *hi, int bins, uint32_t *list, uint64_t *counts,
+               uint64_t *largest) {
+  hipStream_t s = g->stream;
+  const uint64_t n = g->n_rows;
+  for (int b = 0; b < bins; b++) counts[b] = 0;
+  if (largest) *largest = 0;
+  if (n == 0) return SSTG_OK;
+  BinSpec sp{};
+  sp.lo = lo;
+  sp.bins = bins;
+  for (int b = 0; b < bins; b++) sp.hi[b] = hi[b];
+  const uint64_t steps = ceil_div(n, kBinStep);
+  const uint64_t per = ceil_div(steps, kBinBlocks) * kBinStep;
+  const uint32_t blocks = (uint32_t)ceil_div(n, per);
+  uint32_t *cnt = nullptr;
+  uint64_t *tot = nullptr;
+  SSTG_TRY(g->ws.get(kWsBins, (uint64_t)blocks * (kMaxBins + 1), &cnt));
+  SSTG_TRY(g->ws.get(kWsBins + 1, kMaxBins + 1, &tot));
+  uint64_t *host = g->host_ctr_dev ? g->host_ctr_dev + kHostBins : nullptr;
+  const uint64_t seq = host ? ++g->host_seq : 0;
+  SSTG_LAUNCH(k_bins_count, blocks, kScanThreads, 0, s, val, n, per, sp, cnt);
+  SSTG_LAUNCH(k_bins_scan, 1, kBinScanThreads, 0, s, cnt, blocks, bins, tot,
+              host, host ? g->host_ctr_dev + kHostFlag : nullptr, seq);
+  SSTG_LAUNCH(k_bins_place, blocks, kScanThreads, 0, s, val, n, per, sp,
+              (const uint32_t *)cnt, list);
+  const uint64_t *h = g->host_ctr + kHostBins;
+  if (host) {
+    SSTG_TRY(wait_host_flag(g, seq));
+  } else {
+    SSTG_HIP(hipMemcpyAsync(g->host_rb + 16, tot, (bins + 1) * sizeof(uint64_t),
+                            hipMemcpyDeviceToHost, s));
+    SSTG_HIP(hipStreamSynchronize(s));
+    h = g->host_rb + 16;
+  }
+  for (int b = 0; b < bins; b++) counts[b] = h[b];
+  if (largest) *largest = h[bins];
+  return SSTG_OK;
 }
 
 // The radix passes; with pairs, pass 0's histogram comes from the packing

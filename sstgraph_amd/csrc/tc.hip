@@ -20,14 +20,17 @@
 // row u of the store's degree prefix (dag[prefix[u] .. + dplus[u]), sorted by
 // id), so no second scan is needed.
 //
-// Counting stages out(u) in LDS as a linear-probing hash table (load <= 1/4)
-// and streams the lists out(v), v in out(u), through it, with the lanes spread
-// evenly over the concatenated lists.  Six launch tiers by |out(u)|:
-//   [2, 16]    16 lanes per vertex, four vertices per wave
+// Counting stages out(u) in LDS as a hash table and streams the lists out(v),
+// v in out(u), through it.  Launch tiers by |out(u)|:
+//   [2, 16]    four vertices per wave
 //   [17, 64], [65, 128], [129, 256], [257, 512]
-//              one wave per vertex, 1.8 / 3.5 / 7 / 14 KB of LDS
+//              one wave per vertex, 2 / 4 / 8 / 16 KB of table
 //   > 512      one block per vertex; out(u) is hashed in tiles of 4096 ids
-//              and every tile sees all of the lists out(v).
+//              (linear probing, load <= 1/4) and every tile sees all of the
+//              lists out(v).
+// rMat scale 22 (134M triangles, 64M pieces of 64 ids): 7.75 ms with linear
+// tables walked lane by lane, 3.37 ms now, 2.7 of it the counting, which the
+// vector units' issue bounds (80% busy in the [17, 64] tier).
 #include <algorithm>
 
 #include "algo.hpp"
@@ -86,6 +89,27 @@ __device__ __forceinline__ uint32_t hash_has(const uint32_t *table, uint32_t x,
   }
 }
 
+// Two-entry buckets: a probe is one 8-byte LDS read and two compares, with
+// no loop, so a wave's 64 probes end together.  Ids beyond a bucket's two go
+// to a short overflow list that every probe is compared with as well; at four
+// buckets per id or more it is mostly empty (0.6 ids expected at the fullest).
+// kNarrow: ids are below 2^24, so a 24-bit multiply (a quarter of the cost of
+// a 32-bit one) mixes all of their bits.  The result is the bucket's byte
+// offset in a table of 1 << bits buckets: drop = 29 - bits, mask = the
+// offsets' bits.
+template <bool kNarrow>
+__device__ __forceinline__ uint32_t bucket_at(uint32_t x, uint32_t drop,
+                                              uint32_t mask) {
+  return ((kNarrow ? __umul24(x, 0x9E3779u) : x * 0x9E3779B1u) >> drop) & mask;
+}
+
+__device__ __forceinline__ void bucket_insert(uint2 *b, uint32_t x,
+                                              uint32_t *over, uint32_t *nover) {
+  if (atomicCAS(&b->x, kEmpty, x) == kEmpty) return;
+  if (atomicCAS(&b->y, kEmpty, x) == kEmpty) return;
+  over[atomicAdd(nover, 1u)] = x;
+}
+
 // Streams the concatenation of the lists out(v) (list j starts at dag +
 // base[j], its flat range is [pre[j], pre[j+1]), pre[k] = total) through the
 // hash table, P lanes striding the flat index; four loads are issued before
@@ -129,8 +153,10 @@ __device__ __forceinline__ uint64_t probe_lists(const uint32_t *table,
 }
 
 // Orientation, G lanes per row (rows from one degree bin).  Kept neighbours
-// are written in row order by ballot rank inside the lane group.
-template <int G>
+// are written in row order by ballot rank inside the lane group.  Bound by
+// the gathers of the neighbours' degrees: U of a lane's are in flight before
+// the first is used (0.73 -> 0.65 ms over a rMat scale-22 graph).
+template <int G, int U>
 __global__ void __launch_bounds__(256)
     k_tc_orient(DevGraph g, const uint32_t *list, uint64_t count,
                 const uint64_t *prefix, uint32_t *dag, uint32_t *dplus) {
@@ -143,95 +169,171 @@ __global__ void __launch_bounds__(256)
   const uint32_t *row = g.pool + g.off[u];
   uint32_t *out = dag + prefix[u];
   uint32_t c = 0;
-  if (G == 1) {
-    for (uint32_t k = 0; k < du; k++) {
-      const uint32_t v = row[k];
-      if (ranked_above(g.deg[v], v, du, u)) out[c++] = v;
+  const uint32_t lane = lane_id();
+  const uint64_t gmask =
+      (G == 64) ? ~0ull : (((1ull << G) - 1) << (lane & ~(uint32_t)(G - 1)));
+  for (uint32_t k0 = 0; k0 < du; k0 += G * U) {
+    uint32_t v[U], dv[U];
+#pragma unroll
+    for (int j = 0; j < U; j++) {  // past the row's end: its last entry
+      const uint32_t k = k0 + j * G + lig;
+      v[j] = row[k < du ? k : du - 1];
     }
-  } else {
-    const uint32_t lane = lane_id();
-    const uint64_t gmask =
-        (G == 64) ? ~0ull : (((1ull << G) - 1) << (lane & ~(uint32_t)(G - 1)));
-    for (uint32_t k0 = 0; k0 < du; k0 += G) {
-      const uint32_t k = k0 + lig;
-      bool keep = false;
-      uint32_t v = 0;
-      if (k < du) {
-        v = row[k];
-        keep = ranked_above(g.deg[v], v, du, u);
+#pragma unroll
+    for (int j = 0; j < U; j++) dv[j] = g.deg[v[j]];
+#pragma unroll
+    for (int j = 0; j < U; j++) {
+      const bool keep = k0 + j * G + lig < du && ranked_above(dv[j], v[j], du, u);
+      if (G == 1) {
+        if (keep) out[c++] = v[j];
+      } else {
+        const uint64_t m = __ballot(keep) & gmask;
+        if (keep) out[c + mask_rank(m)] = v[j];
+        c += (uint32_t)__popcll(m);
       }
-      const uint64_t m = __ballot(keep) & gmask;
-      if (keep) out[c + mask_rank(m)] = v;
-      c += (uint32_t)__popcll(m);
     }
   }
   if (lig == 0) dplus[u] = c;
 }
 
-// inclusive sum over groups of L lanes (L divides 64)
-template <uint32_t L>
-__device__ __forceinline__ uint32_t group_inclusive_sum(uint32_t v,
-                                                        uint32_t lig) {
-#pragma unroll
-  for (uint32_t o = 1; o < L; o <<= 1) {
-    const uint32_t t = __shfl_up(v, o, L);
-    if (lig >= o) v += t;
-  }
-  return v;
-}
-
-// L lanes per vertex u with 2 <= |out(u)| <= MaxOut, 64 / L vertices per
-// block of one wave, each group with its own LDS table: short lists keep
-// several vertices' setup loads in flight per wave.
-template <uint32_t MaxOut, uint32_t L>
+// NG vertices u per wave with |out(u)| <= MaxOut (NG > 1: at most 64 / NG).
+// Up to 64 lists out(v) at a time are cut into pieces of 64 ids; lane t holds
+// the place and length of the t-th piece, which move to scalar registers one
+// piece at a time.  A piece is then one buffer load from a scalar descriptor
+// whose record count ends with the list, so lanes past its end read 0 with no
+// compare, address or mask of their own, and the probe is a hash, an LDS read
+// and two compares: nine vector and three scalar instructions per 64 ids.
+// (With a ballot, a tail mask and a length test per list, 28 scalar ones
+// bounded it: 5.1 against 3.7 ms for the whole count at rMat scale 22.)  0 is no list's padding but vertex 0
+// as well, so vertex 0 is kept out of the tables: rows are sorted, so it can
+// only be a list's first id, and the vertices that have it look there.
+template <uint32_t MaxOut, uint32_t NG, bool kNarrow>
 __global__ void __launch_bounds__(64)
     k_tc_count_wave(const uint64_t *lbase, const uint32_t *lists,
                     const uint32_t *llen, const uint32_t *list,
                     uint64_t count, unsigned long long *acc) {
   static_assert((MaxOut & (MaxOut - 1)) == 0, "table size must be 2^k");
-  static_assert(4 * MaxOut >= 64 && 64 % L == 0, "group shape");
-  constexpr uint32_t NG = 64 / L;
-  __shared__ uint32_t table[NG][4 * MaxOut];
-  __shared__ uint32_t pre[NG][MaxOut + 1];
-  __shared__ uint64_t base[NG][MaxOut];
+  static_assert(NG == 1 || MaxOut * NG <= 64, "a vertex's lists, one per lane");
+  constexpr uint32_t L = 64 / NG;             // lanes per vertex
+  constexpr uint32_t kTable = 4 * MaxOut;     // buckets per vertex
+  constexpr int kPieces = 8;  // loads issued before their probes (4: 3.87 ms)
+  __shared__ uint4 table4[NG * kTable / 2];
+  __shared__ uint32_t over[NG][MaxOut];
+  __shared__ uint32_t nover[NG];
+  __shared__ uint32_t pre[64], plen[64];
+  __shared__ uint64_t pbase[64];
+  char *tab = reinterpret_cast<char *>(table4);
   const uint32_t lane = threadIdx.x, gi = lane / L, lig = lane % L;
-  uint32_t *tab = table[gi];
-  uint32_t *pr = pre[gi];
-  uint64_t *bs = base[gi];
   uint64_t found = 0;
   for (uint64_t i0 = (uint64_t)blockIdx.x * NG; i0 < count;
        i0 += (uint64_t)gridDim.x * NG) {  // uniform across the block
     const uint64_t i = i0 + gi;
     uint32_t d = 0;
     const uint32_t *row = lists;
-    if (i < count) {
+    if (NG == 1 || i < count) {
       const uint32_t u = list[i];
       d = llen[u];
       row = lists + lbase[u];
     }
-    const uint32_t bits = table_bits(d);
-    for (uint32_t t = lig; t < (1u << bits); t += L) tab[t] = kEmpty;
+    // NG == 1: the table is sized to the vertex (d is uniform then)
+    const uint32_t bits = NG == 1 ? table_bits(d) : __builtin_ctz(kTable);
+    const uint32_t drop = 29 - bits, mask = ((1u << bits) - 1) << 3;
+    const uint32_t tbase = gi * kTable * 8;
+    for (uint32_t t = lane; t < (NG << bits) / 2; t += 64)
+      table4[t] = make_uint4(kEmpty, kEmpty, kEmpty, kEmpty);
+    if (lig == 0) nover[gi] = 0;
     __syncthreads();
-    for (uint32_t j = lig; j < d; j += L) {
-      const uint32_t x = row[j];
-      hash_insert(tab, x, bits);
-      pr[j] = llen[x];
-      bs[j] = lbase[x];
+    bool has0 = false;
+    uint32_t hits = 0;
+    for (uint32_t j0 = 0; j0 < (NG == 1 ? d : 1u); j0 += 64) {
+      // this lane's list, and its id into the table
+      const uint32_t j = NG == 1 ? j0 + lane : lig;
+      uint32_t x = 0, len = 0;
+      uint64_t base = 0;
+      if (j < d) {
+        x = row[j];
+        len = llen[x];
+        base = lbase[x];
+      }
+      has0 |= j == 0 && d > 0 && x == 0;
+      if (NG == 1) {
+        if (j0 == 0) {  // the whole table before the first probe
+          has0 = __any(has0);
+          for (uint32_t k = lane; k < d; k += 64) {
+            const uint32_t y = k == j ? x : row[k];
+            if (y)
+              bucket_insert((uint2 *)(tab + bucket_at<kNarrow>(y, drop, mask)),
+                            y, over[0], &nover[0]);
+          }
+        }
+      } else {
+        has0 = __shfl((int)has0, gi * L, 64);
+        if (x)
+          bucket_insert(
+              (uint2 *)(tab + tbase + bucket_at<kNarrow>(x, drop, mask)), x,
+              over[gi], &nover[gi]);
+      }
+      if (has0 && len && lists[base] == 0) hits++;
+      const uint32_t mine = (len + 63) / 64;
+      const uint32_t incl = wave_inclusive_sum(mine);
+      const uint32_t total = __builtin_amdgcn_readlane(incl, 63);
+      pre[lane] = incl - mine;
+      plen[lane] = len;
+      pbase[lane] = base;
+      __syncthreads();
+      uint32_t any_over = 0;
+#pragma unroll
+      for (uint32_t k = 0; k < NG; k++) any_over |= nover[k];
+      any_over = __builtin_amdgcn_readfirstlane(any_over);
+      for (uint32_t t0 = 0; t0 < total; t0 += 64) {
+        // the lane's piece: the last list that starts at or before it
+        const uint32_t t = t0 + lane;
+        uint32_t s = 0;
+#pragma unroll
+        for (uint32_t step = 32; step > 0; step >>= 1)
+          if (pre[s + step] <= t) s += step;
+        const uint32_t off = (t - pre[s]) * 64;
+        const uint64_t place = t < total ? (uint64_t)(lists + pbase[s] + off) : 0;
+        const uint32_t bytes = t < total ? (plen[s] - off) * 4 : 0;
+        const uint32_t here = total - t0 < 64 ? total - t0 : 64;
+        for (uint32_t p = 0; p < here; p += kPieces) {
+          uint32_t w[kPieces], grp[kPieces];
+#pragma unroll
+          for (int k = 0; k < kPieces; k++) {  // pieces past the last are empty
+            const uint32_t lo = __builtin_amdgcn_readlane((uint32_t)place, p + k);
+            const uint32_t hi =
+                __builtin_amdgcn_readlane((uint32_t)(place >> 32), p + k);
+            const uint32_t nb = __builtin_amdgcn_readlane(bytes, p + k);
+            if (NG > 1) grp[k] = __builtin_amdgcn_readlane(s / L, p + k);
+            w[k] = __builtin_amdgcn_raw_buffer_load_b32(
+                __builtin_amdgcn_make_buffer_rsrc(
+                    (void *)(((uint64_t)hi << 32) | lo), 0, (int)nb, 0x00020000),
+                (int)(lane * 4), 0, 0);
+          }
+          __builtin_amdgcn_sched_barrier(0);  // every load before any wait
+          uint2 e[kPieces];
+#pragma unroll
+          for (int k = 0; k < kPieces; k++) {
+            uint32_t at = bucket_at<kNarrow>(w[k], drop, mask);
+            if (NG > 1) at |= grp[k] * (kTable * 8);
+            e[k] = *(const uint2 *)(tab + at);
+          }
+#pragma unroll
+          for (int k = 0; k < kPieces; k++)
+            hits += (uint32_t)(e[k].x == w[k]) | (uint32_t)(e[k].y == w[k]);
+          if (any_over)
+#pragma unroll
+            for (int k = 0; k < kPieces; k++) {
+              const uint32_t g = NG > 1 ? grp[k] : 0;
+              for (uint32_t o = 0; o < nover[g]; o++)
+                hits += over[g][o] == w[k] ? 1u : 0u;
+            }
+        }
+      }
+      __syncthreads();  // pre, plen and pbase are rewritten
     }
-    __syncthreads();
-    // exclusive scan of the list lengths; pre[d] = total
-    uint32_t carry = 0;
-    for (uint32_t j0 = 0; j0 < d; j0 += L) {
-      const uint32_t j = j0 + lig;
-      const uint32_t x = j < d ? pr[j] : 0;
-      const uint32_t inc = group_inclusive_sum<L>(x, lig);
-      if (j < d) pr[j] = carry + inc - x;
-      carry += __shfl(inc, gi * L + L - 1, 64);
-    }
-    if (lig == 0) pr[d] = carry;
-    __syncthreads();
-    found += probe_lists<L>(tab, bits, pr, bs, lists, carry, lig);
-    __syncthreads();  // table, pre and base are reused by the next vertex
+    found += hits;
+    __syncthreads();  // the tables are reused by the next vertices
   }
   found = wave_sum(found);
   if (lane == 0 && found)
@@ -286,33 +388,9 @@ __global__ void __launch_bounds__(256)
               (unsigned long long)found);
 }
 
-// acc[i * kAccStride] for i < kAccLanes are the spread counters; the slot
-// after them holds the largest list length
+// acc[i * kAccStride] for i < kAccLanes are the spread counters
 __global__ void k_tc_acc_clear(unsigned long long *acc) {
   acc[threadIdx.x * kAccStride] = 0;
-  if (threadIdx.x == 0) acc[kAccLanes * kAccStride] = 0;
-}
-
-// largest len[i]: grid-stride, one atomic per block (few blocks, so the
-// single target address sees few atomics)
-__global__ void __launch_bounds__(256)
-    k_tc_max_len(const uint32_t *len, uint32_t n, unsigned long long *acc) {
-  __shared__ uint32_t wmax[4];
-  uint32_t v = 0;
-  for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < n;
-       i += (uint64_t)gridDim.x * 256)
-    v = len[i] > v ? len[i] : v;
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    const uint32_t t = __shfl_xor(v, o, 64);
-    v = t > v ? t : v;
-  }
-  if ((threadIdx.x & 63) == 0) wmax[threadIdx.x / 64] = v;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int w = 1; w < 4; w++) v = wmax[w] > v ? wmax[w] : v;
-    if (v) atomicMax(&acc[kAccLanes * kAccStride], (unsigned long long)v);
-  }
 }
 
 __global__ void k_tc_acc_sum(unsigned long long *acc) {
@@ -393,6 +471,40 @@ uint32_t grid_for(uint64_t count) {
   return (uint32_t)(count < (1u << 24) ? count : (1u << 24));
 }
 
+// The counting kernel of tier c over the cnt vertices of l.
+template <bool kNarrow>
+void launch_tier(uint32_t c, uint64_t cnt, hipStream_t s, const uint64_t *lbase,
+                 const uint32_t *lists, const uint32_t *llen, const uint32_t *l,
+                 unsigned long long *acc) {
+  const uint32_t grid = grid_for(cnt);
+  switch (c) {
+    case 0:
+      SSTG_LAUNCH((k_tc_count_wave<kTierOut[0], 4, kNarrow>),
+                  grid_for(ceil_div(cnt, 4)), 64, 0, s, lbase, lists, llen, l,
+                  cnt, acc);
+      break;
+    case 1:
+      SSTG_LAUNCH((k_tc_count_wave<kTierOut[1], 1, kNarrow>), grid, 64, 0, s,
+                  lbase, lists, llen, l, cnt, acc);
+      break;
+    case 2:
+      SSTG_LAUNCH((k_tc_count_wave<kTierOut[2], 1, kNarrow>), grid, 64, 0, s,
+                  lbase, lists, llen, l, cnt, acc);
+      break;
+    case 3:
+      SSTG_LAUNCH((k_tc_count_wave<kTierOut[3], 1, kNarrow>), grid, 64, 0, s,
+                  lbase, lists, llen, l, cnt, acc);
+      break;
+    case 4:
+      SSTG_LAUNCH((k_tc_count_wave<kTierOut[4], 1, kNarrow>), grid, 64, 0, s,
+                  lbase, lists, llen, l, cnt, acc);
+      break;
+    default:
+      SSTG_LAUNCH(k_tc_count_block, grid, 256, 0, s, lbase, lists, llen, l, cnt,
+                  acc);
+  }
+}
+
 }  // namespace
 
 int count_list_triangles(sstg_graph *g, const uint64_t *lbase,
@@ -402,62 +514,25 @@ int count_list_triangles(sstg_graph *g, const uint64_t *lbase,
   const uint32_t n = g->n_rows;
   uint32_t *list = nullptr;
   unsigned long long *acc = nullptr;
-  uint8_t *flags = nullptr;
-  uint64_t *tmp = nullptr;
   SSTG_TRY(g->ws.get(kWsTcList, n, &list));
-  SSTG_TRY(g->ws.get(kWsTcAcc, (kAccLanes + 1) * kAccStride, &acc));
-  SSTG_TRY(g->ws.get(kWsAlgo + 24, n, &flags));
-  SSTG_TRY(g->ws.get(kWsAlgo + 25, n, &tmp));
+  SSTG_TRY(g->ws.get(kWsTcAcc, kAccLanes * kAccStride, &acc));
   SSTG_LAUNCH(k_tc_acc_clear, 1, kAccLanes, 0, s, acc);
+  uint32_t hi[kWaveTiers + 1];
+  for (uint32_t c = 0; c < kWaveTiers; c++) hi[c] = kTierOut[c];
+  hi[kWaveTiers] = 0xFFFFFFFFu;
+  uint64_t cnts[kWaveTiers + 1], longest = 0;
+  SSTG_TRY(graph_bins(g, llen, 2, hi, kWaveTiers + 1, list, cnts, &longest));
   // the flat probe index of one vertex (up to 512 lists, or 256 per block
   // step) is 32-bit: lists of 2^23 ids or more go to the caller's fallback
-  SSTG_LAUNCH(k_tc_max_len, (uint32_t)std::min<uint64_t>(ceil_div(n, 256), 512),
-              256, 0, s, llen, n, acc);
-  SSTG_HIP(hipMemcpyAsync(g->host_rb + 17, acc + kAccLanes * kAccStride,
-                          sizeof(uint64_t), hipMemcpyDeviceToHost, s));
-  SSTG_HIP(hipStreamSynchronize(s));
-  if (g->host_rb[17] >= (1u << 23)) return SSTG_E_UNSUPPORTED;
-  for (uint32_t c = 0; c <= kWaveTiers; c++) {
-    const uint32_t lo = c == 0 ? 2 : kTierOut[c - 1] + 1;
-    const uint32_t hi = c < kWaveTiers ? kTierOut[c] : 0xFFFFFFFFu;
-    SSTG_LAUNCH(em::k_bin_flags, ceil_div(n, em::kT), em::kT, 0, s, llen, n,
-                lo, hi, flags);
-    SSTG_TRY(select_flagged_u64(flags, nullptr, n, tmp, g->dev_ctr + 7, g->ws,
-                                kWsPrim, s));
-    SSTG_HIP(hipMemcpyAsync(g->host_rb + 16, g->dev_ctr + 7, sizeof(uint64_t),
-                            hipMemcpyDeviceToHost, s));
-    SSTG_HIP(hipStreamSynchronize(s));
-    const uint64_t cnt = g->host_rb[16];
+  if (longest >= (1u << 23)) return SSTG_E_UNSUPPORTED;
+  const uint32_t *l = list;
+  for (uint32_t c = 0; c <= kWaveTiers; l += cnts[c], c++) {
+    const uint64_t cnt = cnts[c];
     if (!cnt) continue;
-    SSTG_TRY(narrow_u64_to_u32(tmp, cnt, list, s));
-    const uint32_t grid = grid_for(cnt);
-    const uint32_t *l = list;
-    switch (c) {
-      case 0:
-        SSTG_LAUNCH((k_tc_count_wave<kTierOut[0], 16>),
-                    (uint32_t)std::min<uint64_t>(ceil_div(cnt, 4), 1u << 24), 64,
-                    0, s, lbase, lists, llen, l, cnt, acc);
-        break;
-      case 1:
-        SSTG_LAUNCH((k_tc_count_wave<kTierOut[1], 64>), grid, 64, 0, s, lbase,
-                    lists, llen, l, cnt, acc);
-        break;
-      case 2:
-        SSTG_LAUNCH((k_tc_count_wave<kTierOut[2], 64>), grid, 64, 0, s, lbase,
-                    lists, llen, l, cnt, acc);
-        break;
-      case 3:
-        SSTG_LAUNCH((k_tc_count_wave<kTierOut[3], 64>), grid, 64, 0, s, lbase,
-                    lists, llen, l, cnt, acc);
-        break;
-      case 4:
-        SSTG_LAUNCH((k_tc_count_wave<kTierOut[4], 64>), grid, 64, 0, s, lbase,
-                    lists, llen, l, cnt, acc);
-        break;
-      default:
-        SSTG_LAUNCH(k_tc_count_block, grid, 256, 0, s, lbase, lists, llen, l,
-                    cnt, acc);
-    }
+    if (n <= (1u << 24))
+      launch_tier<true>(c, cnt, s, lbase, lists, llen, l, acc);
+    else
+      launch_tier<false>(c, cnt, s, lbase, lists, llen, l, acc);
   }
   SSTG_LAUNCH(k_tc_acc_sum, 1, kAccLanes, 0, s, acc);
   SSTG_HIP(hipMemcpyAsync(g->host_rb, acc, sizeof(uint64_t),
@@ -479,16 +554,16 @@ int tc_oriented(sstg_graph *g, uint64_t *out) {
   SSTG_TRY(g->ws.get(kWsTcDplus, n, &dplus));
   const DevGraph v = g->view();
   if (bins.count[0])
-    SSTG_LAUNCH(k_tc_orient<1>, ceil_div(bins.count[0], 256), 256, 0, s, v,
+    SSTG_LAUNCH((k_tc_orient<1, 4>), ceil_div(bins.count[0], 256), 256, 0, s, v,
                 (const uint32_t *)bins.list[0], bins.count[0], prefix, dag,
                 dplus);
   if (bins.count[1])
-    SSTG_LAUNCH(k_tc_orient<8>, ceil_div(bins.count[1] * 8, 256), 256, 0, s, v,
+    SSTG_LAUNCH((k_tc_orient<8, 4>), ceil_div(bins.count[1] * 8, 256), 256, 0, s, v,
                 (const uint32_t *)bins.list[1], bins.count[1], prefix, dag,
                 dplus);
   for (int b = 2; b < 4; b++)
     if (bins.count[b])
-      SSTG_LAUNCH(k_tc_orient<64>, ceil_div(bins.count[b] * 64, 256), 256, 0,
+      SSTG_LAUNCH((k_tc_orient<64, 4>), ceil_div(bins.count[b] * 64, 256), 256, 0,
                   s, v, (const uint32_t *)bins.list[b], bins.count[b], prefix,
                   dag, dplus);
   return count_list_triangles(g, prefix, dag, dplus, out);
