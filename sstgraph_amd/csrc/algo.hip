@@ -74,36 +74,262 @@ struct Reached {
   }
 };
 
+// ---- top-down levels driven by the device
+// A BFS level of at most a cap of edges is one launch of k_push_level whose
+// grid does not depend on the level, so the host enqueues several levels and
+// reads their counters once.  ctr[k] = edges << 24 | vertices of the batch's
+// k-th frontier, filled by one packed atomic per block of claims, which also
+// orders the claims: each vertex's place in the queue and the running degree
+// sum before it (pre, per frontier, double-buffered, with the row's place in
+// the pool beside it) come from the same value, so the next level's flat edge
+// space needs no pass of its own.  What bounds a level is its chain of
+// dependent memory round trips, some 1 us each behind a kernel boundary:
+// counters, offsets, ids, levels, claims (with the claims' degrees and rows),
+// the packed atomic.  A small level takes 5-8 us where the host-driven one
+// took about 60 (degrees, scan, push, read-back): BFS at rMat scale 16
+// 507 -> 140 us, at scale 24 1.68 -> 1.51 ms.
+constexpr uint32_t kPushT = 512;
+constexpr uint32_t kPushPer = 4;  // most consecutive edges per thread
+constexpr uint32_t kPushTile = kPushT * kPushPer;  // most edges per tile
+constexpr uint32_t kPushGrid = 256;
+constexpr int kPushCountBits = 24;
+constexpr uint64_t kPushCountMask = (1ull << kPushCountBits) - 1;
+constexpr int kPushLevels = 12;  // most levels per batch
+// a frontier of more edges goes back to the host, which may turn bottom-up or
+// launch a push sized to it; a graph of at most kPushAll edges stays here
+constexpr uint64_t kPushCap = 1ull << 20;
+constexpr uint64_t kPushAll = 1ull << 22;
+
+struct PushBatch {
+  unsigned long long *ctr;  // kPushLevels + 1 counters, 3 words of the start
+  uint64_t *start;          // queue index of each frontier
+};
+// A frontier's edge offsets and row places.  A vertex without edges counts as
+// one edge (its row place is kNoRow), so a tile never spans more vertices than
+// edges.
+struct PushFront {
+  uint64_t *pre, *row;
+};
+constexpr uint64_t kNoRow = ~0ull;
+
+// pre: the frontier's offsets, their total behind them
+__global__ void k_push_state(PushBatch pb, uint64_t qs, uint64_t nf,
+                             const uint64_t *pre) {
+  if (threadIdx.x <= kPushLevels)
+    pb.ctr[threadIdx.x] =
+        threadIdx.x == 0 ? (pre[nf] << kPushCountBits) | nf : 0ull;
+  if (threadIdx.x == 0) pb.start[0] = qs;
+}
+
+__global__ void k_front_rows(DevGraph g, const uint32_t *front, uint64_t nf,
+                             uint64_t *row) {
+  const uint64_t i = (uint64_t)blockIdx.x * kT + threadIdx.x;
+  if (i >= nf) return;
+  const uint32_t v = front[i];
+  row[i] = g.deg[v] ? g.off[v] : kNoRow;
+}
+
 // Start of a BFS from src: levels and parents reset, the queue holding src,
-// the visited filter holding only src (threads cover max(n, words)); info
-// gets src's degree and the degree prefix at n / 2 and at n.
+// the visited filter holding only src (threads cover max(n, words)), the step
+// counters cleared and the first batch's frontier set to src; the words after
+// its counters get src's degree and the degree prefix at n / 2 and at n.
 __global__ void k_bfs_start(uint32_t n, uint32_t *level, int32_t *parent,
                             uint32_t src, uint32_t *queue, uint32_t *vis,
                             uint64_t words, const uint32_t *deg,
-                            const uint64_t *prefix,
-                            unsigned long long *info) {
+                            const uint64_t *off, const uint64_t *prefix,
+                            PushBatch pb, PushFront f,
+                            unsigned long long *step, uint32_t nstep) {
   const uint64_t v = (uint64_t)blockIdx.x * kT + threadIdx.x;
   if (v < n) {
     level[v] = (v == src) ? 0u : kInf;
     if (parent) parent[v] = (v == src) ? (int32_t)src : -1;
   }
   if (v < words) vis[v] = (v == (src >> 5)) ? 1u << (src & 31) : 0u;
+  if (v < nstep) step[v] = 0;
+  if (v <= kPushLevels)
+    pb.ctr[v] =
+        v ? 0ull : ((uint64_t)(deg[src] ? deg[src] : 1) << kPushCountBits) | 1;
   if (v == 0) {
     queue[0] = src;
+    pb.start[0] = 0;
+    f.pre[0] = 0;
+    f.row[0] = deg[src] ? off[src] : kNoRow;
+    unsigned long long *info = pb.ctr + kPushLevels + 1;
     info[0] = deg[src];
     info[1] = prefix[n / 2];
     info[2] = prefix[n];
   }
 }
 
-// The tail kernel's starting state, written by a kernel so that a captured
-// launch sequence holds the values themselves.
+// largest i < n with a[i] <= x (a[0] <= x), by one wave
+__device__ __forceinline__ uint32_t wave_segment(const uint64_t *a, uint32_t n,
+                                                 uint64_t x) {
+  const uint32_t lane = lane_id();
+  uint32_t lo = 0, hi = n;  // a[lo] <= x, the answer is below hi
+  while (hi - lo > 1) {     // uniform
+    const uint32_t step = (hi - lo + kWave - 1) / kWave;
+    const uint32_t p = lo + lane * step;
+    const uint64_t m = __ballot(p < hi && a[p < hi ? p : lo] <= x);
+    lo += ((uint32_t)__popcll(m) - 1) * step;  // lane 0 always holds
+    hi = hi < lo + step ? hi : lo + step;
+  }
+  return lo;
+}
+
+// Expands a frontier, flat over its edges, PER consecutive ones per thread.
+// The edge offsets and row places of the tile's frontier vertices go to LDS:
+// of all of them where the frontier is short, else of the range that waves 0
+// and 1 find.  A thread's loads of each kind are issued together, without
+// branches (a lane with nothing to load reads a valid word that it drops; with
+// branches the compiler waited for each load).
+template <uint32_t PER>
+__device__ __forceinline__ void push_tiles(
+    const DevGraph &g, unsigned long long *found, uint32_t nf, uint64_t mf,
+    uint64_t s0, uint32_t L, uint32_t *level, int32_t *parent, uint32_t *queue,
+    const PushFront &cur, const PushFront &next, uint32_t *rel, uint64_t *row) {
+  constexpr uint32_t kTile = kPushT * PER;
+  __shared__ uint32_t ends[2], first;  // first: the vertex of edge e0
+  __shared__ uint64_t wtot[kPushT / kWave], base_lds, into;
+  const uint32_t *front = queue + s0;
+  uint32_t *out = queue + s0 + nf;
+  const uint32_t lane = lane_id(), w = threadIdx.x / kWave;
+  for (uint64_t e0 = (uint64_t)blockIdx.x * kTile; e0 < mf;
+       e0 += (uint64_t)kPushGrid * kTile) {  // uniform across the block
+    const uint64_t e1 = e0 + kTile < mf ? e0 + kTile : mf;
+    uint32_t a = 0, b = nf - 1;
+    if (nf > kTile) {
+      if (w < 2) {
+        const uint32_t s = wave_segment(cur.pre, nf, w ? e1 - 1 : e0);
+        if (lane == 0) ends[w] = s;
+      }
+      __syncthreads();
+      a = ends[0];
+      b = ends[1];  // b - a < kTile: every vertex has an edge
+    }
+    for (uint32_t i = threadIdx.x; i <= b - a; i += kPushT) {
+      const uint64_t p = cur.pre[a + i];
+      const uint64_t q = a + i + 1 < nf ? cur.pre[a + i + 1] : mf;
+      row[i] = cur.row[a + i];
+      rel[i] = p <= e0 ? 0u : p - e0 < kTile ? (uint32_t)(p - e0) : kTile;
+      if (p <= e0 && e0 < q) {
+        first = i;
+        into = e0 - p;
+      }
+    }
+    __syncthreads();
+    const uint32_t t0 = threadIdx.x * PER, te = (uint32_t)(e1 - e0);
+    uint32_t d[PER], x[PER], dg[PER], seg[PER];
+    uint64_t rw[PER];
+    const uint32_t *p[PER];
+    bool ok[PER];
+    {  // each edge's vertex (the last that starts at or before it) and address
+      uint32_t lo = 0, hi = b - a + 1;
+      while (hi - lo > 1) {
+        const uint32_t mid = (lo + hi) >> 1;
+        if (rel[mid] <= t0)
+          lo = mid;
+        else
+          hi = mid;
+      }
+#pragma unroll
+      for (uint32_t j = 0; j < PER; j++) {
+        while (lo < b - a && rel[lo + 1] <= t0 + j) lo++;
+        seg[j] = a + lo;
+        const uint64_t r = row[lo];
+        const uint64_t at = r + (t0 + j) + (lo == first ? into : 0ull) - rel[lo];
+        ok[j] = t0 + j < te && r != kNoRow;
+        p[j] = ok[j] ? g.pool + at : level;
+      }
+    }
+#pragma unroll
+    for (uint32_t j = 0; j < PER; j++)
+      d[j] = *(const __attribute__((address_space(1))) uint32_t *)p[j];
+#pragma unroll
+    for (uint32_t j = 0; j < PER; j++) d[j] = ok[j] ? d[j] : 0u;
+#pragma unroll
+    for (uint32_t j = 0; j < PER; j++) x[j] = level[d[j]];
+#pragma unroll
+    for (uint32_t j = 0; j < PER; j++) ok[j] = ok[j] && x[j] == kInf;
+#pragma unroll
+    for (uint32_t j = 0; j < PER; j++) {  // claims, and what they need
+      const uint32_t y = ok[j] ? d[j] : 0u;
+      dg[j] = g.deg[y];
+      rw[j] = g.off[y];
+    }
+#pragma unroll
+    for (uint32_t j = 0; j < PER; j++)
+      x[j] = ok[j] ? atomicCAS(&level[d[j]], kInf, L + 1) : 0u;
+    uint64_t mine = 0;
+#pragma unroll
+    for (uint32_t j = 0; j < PER; j++) {
+      rw[j] = dg[j] ? rw[j] : kNoRow;
+      dg[j] = dg[j] ? dg[j] : 1u;
+      if (x[j] == kInf) mine += ((uint64_t)dg[j] << kPushCountBits) + 1;
+    }
+    const uint64_t incl = wave_inclusive_sum(mine);
+    if (lane == kWave - 1) wtot[w] = incl;
+    __syncthreads();
+    uint64_t off = incl - mine, all = 0;
+#pragma unroll
+    for (uint32_t i = 0; i < kPushT / kWave; i++) {
+      if (i < w) off += wtot[i];
+      all += wtot[i];
+    }
+    if (threadIdx.x == 0)
+      base_lds = all ? atomicAdd(found, (unsigned long long)all) : 0;
+    __syncthreads();
+    off += base_lds;
+#pragma unroll
+    for (uint32_t j = 0; j < PER; j++)
+      if (x[j] == kInf) {
+        const uint32_t pos = (uint32_t)(off & kPushCountMask);
+        if (parent) parent[d[j]] = (int32_t)front[seg[j]];
+        out[pos] = d[j];
+        next.pre[pos] = off >> kPushCountBits;
+        next.row[pos] = rw[j];
+        off += ((uint64_t)dg[j] << kPushCountBits) + 1;
+      }
+  }
+}
+
+// A level's edges are spread as widely as the grid allows, up to kPushPer per
+// thread: what a compute unit's claims take grows with their number (9,645
+// edges: 53 us in tiles of 4,096, 8.4 in tiles of 512), while every tile adds
+// an atomic to one counter.  cur.pre[nf] is set to the edge count, which a
+// host-sized push over the same frontier reads.
+__global__ void __launch_bounds__(kPushT)
+    k_push_level(DevGraph g, PushBatch pb, int k, uint64_t cap, uint32_t L,
+                 uint32_t *level, int32_t *parent, uint32_t *queue,
+                 PushFront cur, PushFront next) {
+  __shared__ uint32_t rel[kPushTile];  // offsets in the tile
+  __shared__ uint64_t row[kPushTile];
+  const uint64_t c = pb.ctr[k], s0 = pb.start[k];
+  const uint32_t nf = (uint32_t)(c & kPushCountMask);
+  const uint64_t mf = c >> kPushCountBits;
+  if (nf == 0) return;
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    pb.start[k + 1] = s0 + nf;
+    cur.pre[nf] = mf;
+  }
+  if (mf > cap) return;
+  constexpr uint64_t kSpread = (uint64_t)kPushGrid * kPushT;
+  unsigned long long *found = &pb.ctr[k + 1];
+  if (mf <= kSpread)
+    push_tiles<1>(g, found, nf, mf, s0, L, level, parent, queue, cur, next,
+                  rel, row);
+  else if (mf <= 2 * kSpread)
+    push_tiles<2>(g, found, nf, mf, s0, L, level, parent, queue, cur, next,
+                  rel, row);
+  else
+    push_tiles<kPushPer>(g, found, nf, mf, s0, L, level, parent, queue, cur,
+                         next, rel, row);
+}
+
+// The tail kernel's starting state (a kernel argument, so that a captured
+// launch holds the values themselves); it leaves its final state in memory.
 struct TailState {
   uint64_t w[7];
 };
-__global__ void k_tail_state(uint64_t *st, TailState t) {
-  if (threadIdx.x < 7) st[threadIdx.x] = t.w[threadIdx.x];
-}
 
 __global__ void k_level_dist(const uint32_t *level, uint32_t n, int32_t *out) {
   uint64_t v = (uint64_t)blockIdx.x * kT + threadIdx.x;
@@ -496,26 +722,24 @@ struct BfsRun {
 // degree sum of the current frontier; ends[k] = end of the frontier found by
 // the k-th level run.
 constexpr uint32_t kTailThreads = 1024;
-constexpr uint32_t kTailFrontier = 16384;
-constexpr uint32_t kTailEdges = 1u << 17;
+constexpr uint32_t kTailFrontier = 4096;
+constexpr uint32_t kTailEdges = 4096;
 constexpr uint32_t kTailLevels = 1024;
 constexpr uint32_t kTailPer = kTailFrontier / kTailThreads;
 constexpr uint32_t kTailBatch = 4;
-// a source of larger degree starts with a grid-wide push instead
-constexpr uint32_t kTailStartEdges = 2048;
 
 __global__ void __launch_bounds__(kTailThreads)
     k_bfs_tail(DevGraph g, uint32_t *level, int32_t *parent, uint32_t *queue,
-               uint64_t *state, uint64_t *ends) {
+               TailState from, uint64_t *state, uint64_t *ends) {
   __shared__ uint32_t pre[kTailFrontier + 1];
   __shared__ uint32_t wsum[kTailThreads / kWave];
   __shared__ uint32_t s_next;
   __shared__ unsigned long long s_edges;
   const uint32_t tid = threadIdx.x, lane = lane_id(), wave = tid / kWave;
-  uint64_t head = state[0];
-  uint32_t cnt = (uint32_t)state[1];
-  uint32_t L = (uint32_t)state[2];
-  uint64_t prev = state[5], found_edges = 0, cur_edges = state[6];
+  uint64_t head = from.w[0];
+  uint32_t cnt = (uint32_t)from.w[1];
+  uint32_t L = (uint32_t)from.w[2];
+  uint64_t prev = from.w[5], found_edges = 0, cur_edges = from.w[6];
   uint32_t k = 0;
   while (cnt > 0 && k < kTailLevels) {  // cnt and k are block-uniform
     // exclusive prefix of the frontier's degrees (kTailPer per thread)
@@ -635,17 +859,49 @@ static int bfs_core(sstg_graph *g, uint32_t src, uint32_t *level,
   ctx.log = log;
   uint32_t *queue = order;
   if (!queue) SSTG_TRY(ws.get(kWsAlgo + 10, (uint64_t)n + 1, &queue));
-  unsigned long long *info = ctx.ctrs + 2 * em::kStepCtrs;
+  // device-driven levels: alternate frontiers' offsets and rows, of which the
+  // current one's are in pre_cur when it is pre_front
+  const uint64_t push_cap = g->m <= kPushAll ? ~0ull : kPushCap;
+  const int push_steps = g->m <= kPushAll ? kPushLevels : kPushLevels / 3;
+  const uint64_t pre_n =
+      std::min<uint64_t>(n, g->m <= kPushAll ? kPushAll : kPushCap) + 2;
+  PushFront pre_buf[2], pre_cur;
+  PushBatch pb;
+  for (int i = 0; i < 2; i++) {
+    SSTG_TRY(ws.get(kWsPush + i, 2 * pre_n, &pre_buf[i].pre));
+    pre_buf[i].row = pre_buf[i].pre + pre_n;
+  }
+  SSTG_TRY(ws.get(kWsPush + 2, kPushLevels + 1 + 3, &pb.ctr));
+  SSTG_TRY(ws.get(kWsPush + 3, kPushLevels + 2, &pb.start));
+  const uint32_t *pre_front = queue;
+  pre_cur = pre_buf[0];
   SSTG_LAUNCH(k_bfs_start, blocks(std::max<uint64_t>(n, ctx.words)), kT, 0, s,
               n, level, parent, src, queue, ctx.vis, ctx.words,
-              (const uint32_t *)g->deg, prefix, info);
-  // the source's degree, and the degree mass of the upper half of the ids
-  // against the whole (rows are sorted by id, so when the high ids carry
-  // more edges -- as in the reference's rMat, whose hubs have mostly 1
-  // bits -- a frontier vertex is met sooner from a row's end)
-  SSTG_TRY(read_back(g, log, g->host_rb + 8, info, 3 * sizeof(uint64_t)));
-  const uint32_t src_deg = (uint32_t)g->host_rb[8];
-  ctx.rev = 2 * g->host_rb[9] < g->host_rb[10];
+              (const uint32_t *)g->deg, (const uint64_t *)g->off, prefix, pb,
+              pre_buf[0], ctx.ctrs, (uint32_t)(2 * em::kStepCtrs));
+  // one batch of push levels from frontier pre_cur (level L), its counters
+  // and the start's three words read back into c
+  PushFront cur[kPushLevels + 1];
+  uint64_t c[kPushLevels + 1 + 3];
+  auto push_batch = [&](uint32_t L) -> int {
+    cur[0] = pre_cur;
+    for (int k = 0; k < push_steps; k++) {
+      cur[k + 1] = cur[k].pre == pre_buf[0].pre ? pre_buf[1] : pre_buf[0];
+      SSTG_LAUNCH(k_push_level, kPushGrid, kPushT, 0, s, g->view(), pb, k,
+                  push_cap, L + (uint32_t)k, level, parent, queue, cur[k],
+                  cur[k + 1]);
+    }
+    return read_back(g, log, c, pb.ctr, sizeof(c));
+  };
+  // the first batch starts before the host knows the source's degree, and
+  // does nothing if that is over the cap; with it come the degree mass of the
+  // upper half of the ids and the whole (rows are sorted by id, so when the
+  // high ids carry more edges -- as in the reference's rMat, whose hubs have
+  // mostly 1 bits -- a frontier vertex is met sooner from a row's end)
+  SSTG_TRY(push_batch(0));
+  bool batch_done = true;
+  const uint32_t src_deg = (uint32_t)c[kPushLevels + 1];
+  ctx.rev = 2 * c[kPushLevels + 2] < c[kPushLevels + 3];
   uint64_t qs = 0, nf = 1, mf = src_deg;
   uint64_t explored = src_deg;  // edges of visited vertices
   bool bottom_up = false;
@@ -679,17 +935,15 @@ static int bfs_core(sstg_graph *g, uint32_t src, uint32_t *level,
       SSTG_TRY(frontier_prefix(g, ctx, queue + qs, nf, &mf));
       explored += mf;
     }
-    if (!want_bu && nf <= kTailFrontier && mf <= kTailEdges &&
-        (L > 0 || mf <= kTailStartEdges)) {
+    if (!want_bu && L > 0 && nf <= kTailFrontier && mf <= kTailEdges) {
       // the remaining top-down levels in one block (k_bfs_tail)
       uint64_t *st = nullptr, *ends = nullptr;
       SSTG_TRY(ws.get(kWsAlgo + 8, 8, &st));
       SSTG_TRY(ws.get(kWsAlgo + 9, kTailLevels, &ends));
       uint64_t *h = g->host_rb + 48;  // pinned staging
       const TailState t0{{qs, nf, L, 0, 0, prev_nf, mf}};
-      SSTG_LAUNCH(k_tail_state, 1, kWave, 0, s, st, t0);
       SSTG_LAUNCH(k_bfs_tail, 1, kTailThreads, 0, s, g->view(), level, parent,
-                  queue, st, ends);
+                  queue, t0, st, ends);
       SSTG_TRY(read_back(g, log, h, st, 7 * sizeof(uint64_t)));
       const uint64_t levels_run = h[3];
       if (run && levels_run) {
@@ -716,8 +970,61 @@ static int bfs_core(sstg_graph *g, uint32_t src, uint32_t *level,
       bottom_up = false;
       continue;
     }
+    if (batch_done || (!want_bu && mf <= push_cap && nf <= kPushCountMask)) {
+      if (!batch_done) {
+        if (pre_front != queue + qs) {
+          // offsets from a bottom-up step's end serve as they are: its
+          // vertices all have edges
+          if (ctx.fpre_front != queue + qs || ctx.fpre_n != nf || !symmetric)
+            SSTG_TRY(frontier_prefix(g, ctx, queue + qs, nf, nullptr, 1));
+          ctx.fpre_front = nullptr;
+          pre_cur.pre = ctx.fpre;
+          SSTG_TRY(ws.get(kWsPush + 4, nf, &pre_cur.row));
+          SSTG_LAUNCH(k_front_rows, blocks(nf), kT, 0, s, g->view(),
+                      (const uint32_t *)(queue + qs), nf, pre_cur.row);
+        }
+        SSTG_LAUNCH(k_push_state, 1, kWave, 0, s, pb, qs, nf,
+                    (const uint64_t *)pre_cur.pre);
+        SSTG_TRY(push_batch(L));
+      }
+      batch_done = false;
+      int k = 0;
+      while (k < push_steps && nf > 0 && mf <= push_cap) {  // expanded on the device
+        k++;
+        qs += nf;
+        prev_nf = nf;
+        nf = c[k] & kPushCountMask;
+        mf = c[k] >> kPushCountBits;
+        explored += mf;
+        L++;
+        if (run) run->level_start.push_back(qs + nf);
+      }
+      vis_stale = vis_stale || k > 0;
+      bottom_up = false;
+      // after all its steps the last frontier's total is still to be written
+      pre_front = k < push_steps ? queue + qs : nullptr;
+      pre_cur = cur[k];
+      if (k < push_steps && symmetric) {
+        // stopped over the cap: offsets complete for a push (a vertex without
+        // edges, which only a graph with one-directional edges reaches, would
+        // count as one)
+        ctx.fpre = cur[k].pre;
+        ctx.fpre_front = queue + qs;
+        ctx.fpre_n = nf;
+      }
+      if (verbose) {
+        const auto t1 = std::chrono::steady_clock::now();
+        std::fprintf(stderr, "bfs %d levels on the device, next %llu  %.3f ms\n",
+                     k, (unsigned long long)nf,
+                     std::chrono::duration<double, std::milli>(t1 - t_level)
+                         .count());
+        t_level = t1;
+      }
+      continue;
+    }
     EdgeMapResult res;
     uint32_t *next = queue + qs + nf;
+    pre_front = nullptr;
     if (want_bu) {
       SSTG_TRY(edge_map_dense(g, ctx, BfsPull{level, parent, L + 1},
                               LevelIs{level, L}, next, &res));

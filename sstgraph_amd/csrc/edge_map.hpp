@@ -43,8 +43,12 @@ inline int read_back(sstg_graph *g, ReadLog *log, void *dst, const void *src,
     log->pos += nw;
     return SSTG_OK;
   }
-  SSTG_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, g->stream));
-  SSTG_HIP(hipStreamSynchronize(g->stream));
+  if (bytes % 8 == 0) {
+    SSTG_TRY(read_words(g, src, nw, dst));
+  } else {
+    SSTG_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, g->stream));
+    SSTG_HIP(hipStreamSynchronize(g->stream));
+  }
   if (log && log->mode == 1) {
     const size_t at = log->words.size();
     log->words.resize(at + nw, 0);
@@ -90,15 +94,10 @@ __global__ void k_clear_u32(uint32_t *p, uint64_t n) {
   if (i < n) p[i] = 0;
 }
 
-__global__ void k_clear_u64(unsigned long long *p, uint64_t n) {
-  uint64_t i = (uint64_t)blockIdx.x * kT + threadIdx.x;
-  if (i < n) p[i] = 0;
-}
-
 __global__ void k_frontier_degrees(DevGraph g, const uint32_t *q, uint64_t nq,
-                                   uint64_t *out) {
+                                   uint32_t least, uint64_t *out) {
   uint64_t i = (uint64_t)blockIdx.x * kT + threadIdx.x;
-  if (i < nq) out[i] = g.deg[q[i]];
+  if (i < nq) out[i] = max(g.deg[q[i]], least);
   if (i == nq) out[nq] = 0;
 }
 
@@ -532,20 +531,15 @@ struct OnLevel {
 }  // namespace em
 
 // Buffers of a BFS: the frontier bitmap and the visited filter at slot and
-// slot + 1, the frontier degree prefix at slot + 2; both counter sets (and
-// kCtxExtra words after them) cleared by a kernel, which a captured launch
-// sequence can hold.
-constexpr int kCtxExtra = 8;
+// slot + 1, the frontier degree prefix at slot + 2; the caller clears both
+// counter sets in its first kernel.
 inline int edge_map_ctx(sstg_graph *g, EdgeMapCtx *ctx, int slot) {
   ctx->words = ((uint64_t)g->n_rows + 31) / 32 + 1;
   ctx->slot = slot;
   SSTG_TRY(g->ws.get(slot + 0, ctx->words, &ctx->bm));
   SSTG_TRY(g->ws.get(slot + 1, ctx->words, &ctx->vis));
-  SSTG_TRY(g->ws.get(kWsBottomUp + 2, 2 * em::kStepCtrs + kCtxExtra,
-                     &ctx->ctrs));
+  SSTG_TRY(g->ws.get(kWsBottomUp + 2, 2 * em::kStepCtrs, &ctx->ctrs));
   ctx->parity = 0;
-  SSTG_LAUNCH(em::k_clear_u64, 1, em::kT, 0, g->stream, ctx->ctrs,
-              (uint64_t)(2 * em::kStepCtrs + kCtxExtra));
   return SSTG_OK;
 }
 
@@ -581,15 +575,15 @@ inline int step_counters(sstg_graph *g, EdgeMapCtx &ctx, int k) {
 }
 
 // Exclusive degree prefix of the frontier front[0..nf) into ctx.fpre
-// (nf + 1 entries); with total given, the degree sum is read back into it
-// (one copy, one wait).
+// (nf + 1 entries), each degree taken as at least `least`; with total given,
+// the degree sum is read back into it (one wait).
 inline int frontier_prefix(sstg_graph *g, EdgeMapCtx &ctx,
                            const uint32_t *front, uint64_t nf,
-                           uint64_t *total) {
+                           uint64_t *total, uint32_t least = 0) {
   hipStream_t s = g->stream;
   SSTG_TRY(g->ws.get(ctx.slot + 2, nf + 1, &ctx.fpre));
   SSTG_LAUNCH(em::k_frontier_degrees, ceil_div(nf + 1, em::kT), em::kT, 0, s,
-              g->view(), front, nf, ctx.fpre);
+              g->view(), front, nf, least, ctx.fpre);
   SSTG_TRY(scan_exclusive_u64(ctx.fpre, ctx.fpre, nf + 1, nullptr, g->ws,
                               kWsPrim2, s));
   ctx.fpre_front = front;

@@ -114,9 +114,11 @@ int graph_alloc(sstg_graph *g);
 void graph_free(sstg_graph *g);
 // host_ctr holds kHostCtrSlots words: the counter blocks from 0 and, at
 // kHostFlag, the sequence number a kernel writes after them
-constexpr int kHostCtrSlots = 64;
+constexpr int kHostCtrSlots = 512;
 constexpr int kHostFlag = 24;
-constexpr int kHostBins = 32;  // graph_bins: the totals
+constexpr int kHostBins = 32;   // graph_bins: the totals
+constexpr int kHostWords = 64;  // read_words: up to kReadWords words
+constexpr int kReadWords = kHostCtrSlots - kHostWords;
 
 // Waits until the device has written seq to host_ctr[kHostFlag] (spinning on
 // the mapped word, which arrives as soon as the kernel writes it rather than
@@ -124,6 +126,9 @@ constexpr int kHostBins = 32;  // graph_bins: the totals
 // reads after it.  Falls back to a stream synchronisation when the graph has
 // no mapped block or the flag has not come within 100 ms.
 int wait_host_flag(sstg_graph *g, uint64_t seq);
+// nw words of device memory to host memory, once the stream's earlier work is
+// done.
+int read_words(sstg_graph *g, const void *src, size_t nw, void *dst);
 
 int graph_update(sstg_graph *g, const uint32_t *src, const uint32_t *dst,
                  uint64_t n, bool insert, bool skip_self, bool device_ptrs);
@@ -243,6 +248,7 @@ enum : int {
   kWsSmallRows = 147,
   kWsSmallFound = 149,  // small updates: each pair's row search
   kWsRebuild = 150,     // 150..152 pool rebuild: capacities, offsets, prefix
+  kWsPush = 155,        // 155..159 device-driven BFS levels
   kWsBins = 153,        // 153, 154 graph_bins: block counts, totals
 };
 

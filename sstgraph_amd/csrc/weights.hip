@@ -377,7 +377,7 @@ int algo_bf_weighted(sstg_graph *g, uint32_t src, int32_t *dist) {
   uint64_t nf = 1;
   for (uint32_t round = 0; round < n && nf; round++) {
     SSTG_LAUNCH(em::k_frontier_degrees, nblocks(nf + 1), kT, 0, s, g->view(),
-                (const uint32_t *)q, nf, fpre);
+                (const uint32_t *)q, nf, 0u, fpre);
     SSTG_TRY(scan_exclusive_u64(fpre, fpre, nf + 1, g->dev_ctr + 8, g->ws,
                                 kWsPrim, s));
     SSTG_HIP(hipMemcpyAsync(g->host_rb + 19, g->dev_ctr + 8, sizeof(uint64_t),

@@ -1,0 +1,86 @@
+"""BFS where its top-down levels change hands: device-driven batches, the
+one-block tail and host-sized pushes, with frontiers around the tile and cap
+sizes, chains longer than any batch, and vertices without out-edges."""
+import numpy as np
+import pytest
+
+import sstgraph_amd as S
+from oracle import oracle as O
+from tests.gpu_common import need_gpu, say
+
+pytestmark = pytest.mark.gpu
+EMV = S.EdgeMapVertexMap
+
+
+def _check(n, s, d, sources, sym=True):
+    s, d = np.asarray(s, np.uint32), np.asarray(d, np.uint32)
+    if sym:
+        s, d = np.concatenate([s, d]), np.concatenate([d, s])
+    og = O.Graph(n)
+    og.insert_batch(s, d)
+    off, cols = og.csr()
+    g = S.SparseMatrixV(n)
+    g.insert_batch(s, d)
+    for src in sources:
+        say("bfs", n, len(cols), src)
+        want, _ = O.bfs(off, cols, src)
+        parent, level = EMV.BFS(g, src, levels=True)
+        assert np.array_equal(level, want)
+        reached = want != S.UNREACHED
+        assert np.array_equal(parent >= 0, reached) and parent[src] == src
+        v = np.nonzero(reached)[0]
+        v = v[v != src]
+        p = parent[v]
+        assert np.all(want[p] + 1 == want[v])
+        # every tree edge is an edge: its key is among the graph's
+        keys = np.repeat(np.arange(n, dtype=np.uint64), np.diff(off).astype(np.int64))
+        keys = keys * np.uint64(n) + cols
+        assert np.isin(p.astype(np.uint64) * np.uint64(n) + v.astype(np.uint64),
+                       keys).all()
+
+
+@pytest.mark.parametrize("leaves", [1, 511, 512, 513, 2047, 2049, 131071,
+                                    131073, 262145])
+@pytest.mark.parametrize("sym", [True, False])
+def test_stars_joined(leaves, sym):
+    """A source, its leaves, and a second hub behind them: frontiers of 1,
+    `leaves` and 1 vertices (leaves without out-edges when directed)."""
+    need_gpu()
+    n = leaves + 3
+    leaf = np.arange(1, leaves + 1)
+    s = np.concatenate([0 * leaf, leaf[::3], [leaves + 1]])
+    d = np.concatenate([leaf, 0 * leaf[::3] + leaves + 1, [leaves + 2]])
+    _check(n, s, d, [0, 1, leaves + 1, leaves + 2], sym)
+
+
+@pytest.mark.parametrize("n", [2, 13, 14, 1500, 5000])
+def test_chain(n):
+    need_gpu()
+    v = np.arange(n - 1)
+    _check(n, v, v + 1, [0, n // 2, n - 1])
+
+
+@pytest.mark.parametrize("degree", [1 << 20, (1 << 20) + 1])
+def test_second_level_at_the_cap(degree):
+    """In a graph too large to stay on the device, a second frontier of the
+    cap's edges, or one more, and a third that reads its offsets."""
+    need_gpu()
+    hubs, n = 64, 1 << 21
+    rng = np.random.default_rng(degree)
+    per = np.full(hubs, (degree - hubs) // hubs)
+    per[: degree - hubs - per.sum()] += 1  # with the source's edge: `degree`
+    s = np.repeat(np.arange(1, hubs + 1), per)
+    d = hubs + 1 + np.concatenate([rng.permutation(n - hubs - 1)[:k] for k in per])
+    extra = rng.integers(hubs + 1, n, (2, 2 << 20))
+    s = np.concatenate([np.zeros(hubs, int), s, extra[0]])
+    d = np.concatenate([np.arange(1, hubs + 1), d, extra[1]])
+    _check(n, s, d, [0])
+
+
+@pytest.mark.parametrize("sym", [True, False])
+def test_random_graph_any_source(sym):
+    need_gpu()
+    n = 300001
+    rng = np.random.default_rng(3)
+    s, d = rng.integers(0, n, 2 * n), rng.integers(0, n, 2 * n)
+    _check(n, s, d, [0, 7, n - 1], sym)
