@@ -3,6 +3,8 @@
 // kernel profiler, error notes).
 #include <cstdlib>
 
+#include <unordered_map>
+
 #include "algo.hpp"
 #include "graph.hpp"
 
@@ -97,6 +99,113 @@ void Profiler::reset() {
   acc.clear();
 }
 
+// ------------------------------------------------------- device memory
+namespace {
+struct DevBlock {
+  void *p;
+  size_t bytes;
+  int dev;
+};
+// Never destroyed: graphs may be dropped while the process's statics go.
+struct DevCache {
+  std::mutex mu;
+  std::vector<DevBlock> idle;                   // newest last
+  std::unordered_map<void *, DevBlock> in_use;  // blocks dev_alloc handed out
+  size_t idle_bytes = 0;
+};
+DevCache &dev_cache() {
+  static DevCache *c = new DevCache();
+  return *c;
+}
+}  // namespace
+
+hipError_t dev_alloc(void **out, size_t bytes, size_t *got) {
+  DevCache &c = dev_cache();
+  *out = nullptr;
+  int dev = 0;
+  hipError_t e = hipGetDevice(&dev);
+  if (e != hipSuccess) return e;
+  if (!bytes) bytes = 1;
+  {
+    std::lock_guard<std::mutex> lk(c.mu);
+    size_t best = c.idle.size();
+    for (size_t i = 0; i < c.idle.size(); i++) {
+      const DevBlock &b = c.idle[i];
+      if (b.dev == dev && b.bytes >= bytes && b.bytes - bytes <= bytes / 2 &&
+          (best == c.idle.size() || b.bytes < c.idle[best].bytes))
+        best = i;
+    }
+    if (best < c.idle.size()) {
+      const DevBlock b = c.idle[best];
+      c.idle.erase(c.idle.begin() + (ptrdiff_t)best);
+      c.idle_bytes -= b.bytes;
+      c.in_use[b.p] = b;
+      *out = b.p;
+      if (got) *got = b.bytes;
+      return hipSuccess;
+    }
+  }
+  e = hipMalloc(out, bytes);
+  if (e == hipErrorOutOfMemory) {
+    (void)hipGetLastError();
+    dev_trim();
+    e = hipMalloc(out, bytes);
+  }
+  if (e != hipSuccess) {
+    *out = nullptr;
+    return e;
+  }
+  std::lock_guard<std::mutex> lk(c.mu);
+  c.in_use[*out] = DevBlock{*out, bytes, dev};
+  if (got) *got = bytes;
+  return hipSuccess;
+}
+
+void dev_free(void *p) {
+  if (!p) return;
+  DevCache &c = dev_cache();
+  std::vector<void *> back;
+  {
+    std::lock_guard<std::mutex> lk(c.mu);
+    auto it = c.in_use.find(p);
+    if (it == c.in_use.end() || it->second.bytes > kDevKeep / 2) {
+      if (it != c.in_use.end()) c.in_use.erase(it);
+      back.push_back(p);
+    } else {
+      c.idle.push_back(it->second);
+      c.idle_bytes += it->second.bytes;
+      c.in_use.erase(it);
+      while (c.idle_bytes > kDevKeep) {  // the oldest first
+        back.push_back(c.idle.front().p);
+        c.idle_bytes -= c.idle.front().bytes;
+        c.idle.erase(c.idle.begin());
+      }
+    }
+  }
+  for (void *q : back) (void)hipFree(q);
+}
+
+void dev_release(void *p) {
+  if (!p) return;
+  DevCache &c = dev_cache();
+  {
+    std::lock_guard<std::mutex> lk(c.mu);
+    c.in_use.erase(p);
+  }
+  (void)hipFree(p);
+}
+
+void dev_trim() {
+  DevCache &c = dev_cache();
+  std::vector<DevBlock> back;
+  {
+    std::lock_guard<std::mutex> lk(c.mu);
+    back.swap(c.idle);
+    c.idle_bytes = 0;
+  }
+  for (const DevBlock &b : back) (void)hipFree(b.p);
+}
+
 // ----------------------------------------------------------- workspace
 int Workspace::get(int slot, size_t bytes, void **out) {
   if (slot < 0) return SSTG_E_INVAL;
@@ -119,7 +228,7 @@ int Workspace::get(int slot, size_t bytes, void **out) {
   if (s.bytes < bytes) {
     if (s.p) {
       if (stream) hipStreamSynchronize(stream);
-      hipFree(s.p);
+      dev_free(s.p);
       total -= s.bytes;
       s.p = nullptr;
       s.bytes = 0;
@@ -127,11 +236,11 @@ int Workspace::get(int slot, size_t bytes, void **out) {
     size_t want = bytes + bytes / 4;
     want = (want + 4095) & ~(size_t)4095;
     void *p = nullptr;
-    hipError_t e = hipMalloc(&p, want);
+    hipError_t e = dev_alloc(&p, want, &want);
     if (e != hipSuccess) {
       (void)hipGetLastError();
       want = (bytes + 4095) & ~(size_t)4095;
-      e = hipMalloc(&p, want);
+      e = dev_alloc(&p, want, &want);
       if (e != hipSuccess) {
         note_hip_error(e, "workspace hipMalloc", __FILE__, __LINE__);
         return SSTG_E_NOMEM;
@@ -148,8 +257,7 @@ int Workspace::get(int slot, size_t bytes, void **out) {
 
 void Workspace::release_all() {
   if (stream) hipStreamSynchronize(stream);
-  for (auto &s : slots)
-    if (s.p) hipFree(s.p);
+  for (auto &s : slots) dev_free(s.p);
   slots.clear();
   total = 0;
   generation++;
@@ -710,6 +818,7 @@ int sstg_device_synchronize(void) {
 }
 
 int sstg_mem_info(uint64_t *free_bytes, uint64_t *total_bytes) {
+  dev_trim();  // memory kept for reuse counts as free
   size_t f = 0, t = 0;
   SSTG_HIP(hipMemGetInfo(&f, &t));
   if (free_bytes) *free_bytes = f;

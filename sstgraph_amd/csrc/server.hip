@@ -176,10 +176,10 @@ uint64_t store_bytes(uint32_t n, uint64_t pool_cap) {
 }
 
 void free_set_arrays(StoreSet &t) {
-  hipFree(t.off);
-  hipFree(t.deg);
-  hipFree(t.cap);
-  hipFree(t.pool);
+  dev_release(t.off);
+  dev_release(t.deg);
+  dev_release(t.cap);
+  dev_release(t.pool);
 }
 
 // Result buffers are recycled by size: hipFree would wait for the whole
@@ -721,7 +721,7 @@ void view_free(sstg_graph *v) {
   pagerank_release(v);
   v->ws.release_all();
   hipFree(v->dev_ctr);
-  hipFree(v->deg_prefix);
+  dev_release(v->deg_prefix);
   if (v->host_rb) hipHostFree(v->host_rb);
   if (v->stream) hipStreamDestroy(v->stream);
   // the store arrays belong to the served graph
@@ -762,6 +762,7 @@ int sstg_server_create(sstg_graph *g, uint32_t slots, uint64_t hbm_budget,
   }
   if (S->maintain && sym) S->tc_chain[g->version] = 0;
   size_t free_b = 0, total_b = 0;
+  dev_trim();  // memory kept for reuse counts as free
   if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) {
     hipStreamDestroy(S->fetch_stream);
     delete S;

@@ -1004,13 +1004,13 @@ inline uint64_t chunk_blocks(uint64_t n) {
 
 int graph_alloc(sstg_graph *g) {
   uint64_t n = g->n_rows ? g->n_rows : 1;
-  SSTG_HIP(hipMalloc(&g->off, n * sizeof(uint64_t)));
-  SSTG_HIP(hipMalloc(&g->deg, n * sizeof(uint32_t)));
-  SSTG_HIP(hipMalloc(&g->cap, n * sizeof(uint32_t)));
+  SSTG_HIP(dev_alloc(&g->off, n * sizeof(uint64_t)));
+  SSTG_HIP(dev_alloc(&g->deg, n * sizeof(uint32_t)));
+  SSTG_HIP(dev_alloc(&g->cap, n * sizeof(uint32_t)));
   SSTG_HIP(hipMemsetAsync(g->off, 0, n * sizeof(uint64_t), g->stream));
   SSTG_HIP(hipMemsetAsync(g->deg, 0, n * sizeof(uint32_t), g->stream));
   SSTG_HIP(hipMemsetAsync(g->cap, 0, n * sizeof(uint32_t), g->stream));
-  SSTG_HIP(hipMalloc(&g->dev_ctr, kCtrCount * sizeof(uint64_t)));
+  SSTG_HIP(dev_alloc(&g->dev_ctr, kCtrCount * sizeof(uint64_t)));
   SSTG_HIP(hipHostMalloc(&g->host_rb, 64 * sizeof(uint64_t),
                          hipHostMallocDefault));
   SSTG_HIP(hipHostMalloc(&g->host_ctr, kHostCtrSlots * sizeof(uint64_t),
@@ -1026,12 +1026,12 @@ void graph_free(sstg_graph *g) {
   if (g->stream) hipStreamSynchronize(g->stream);
   pagerank_release(g);
   weights_free(g);
-  hipFree(g->off);
-  hipFree(g->deg);
-  hipFree(g->cap);
-  hipFree(g->pool);
-  hipFree(g->dev_ctr);
-  hipFree(g->deg_prefix);
+  dev_free(g->off);
+  dev_free(g->deg);
+  dev_free(g->cap);
+  dev_free(g->pool);
+  dev_free(g->dev_ctr);
+  dev_free(g->deg_prefix);
   if (g->host_rb) hipHostFree(g->host_rb);
   if (g->host_ctr) hipHostFree(g->host_ctr);
   g->ws.release_all();
@@ -1067,11 +1067,11 @@ static int rebuild_impl(sstg_graph *g, uint64_t extra, bool recompute) {
   uint64_t want = total + extra;
   uint64_t new_cap_elems = want + want / 4 + (1u << 20);
   uint32_t *new_pool = nullptr;
-  hipError_t e = hipMalloc(&new_pool, new_cap_elems * sizeof(uint32_t));
+  hipError_t e = dev_alloc(&new_pool, new_cap_elems * sizeof(uint32_t));
   if (e != hipSuccess) {
     (void)hipGetLastError();
     new_cap_elems = want + 1024;
-    SSTG_HIP(hipMalloc(&new_pool, new_cap_elems * sizeof(uint32_t)));
+    SSTG_HIP(dev_alloc(&new_pool, new_cap_elems * sizeof(uint32_t)));
   }
   if (g->m) {
     SSTG_TRY(g->ws.get(kWsRebuild + 2, n + 1, &prefix));
@@ -1084,7 +1084,7 @@ static int rebuild_impl(sstg_graph *g, uint64_t extra, bool recompute) {
                 (const uint64_t *)new_off);
   }
   SSTG_HIP(hipStreamSynchronize(s));
-  hipFree(g->pool);
+  dev_free(g->pool);
   g->pool = new_pool;
   g->pool_cap = new_cap_elems;
   g->pool_tail = total;
@@ -1454,7 +1454,7 @@ int graph_update(sstg_graph *g, const uint32_t *src, const uint32_t *dst,
 
 int graph_degree_prefix(sstg_graph *g, const uint64_t **out) {
   if (!g->deg_prefix) {
-    SSTG_HIP(hipMalloc(&g->deg_prefix, ((uint64_t)g->n_rows + 1) *
+    SSTG_HIP(dev_alloc(&g->deg_prefix, ((uint64_t)g->n_rows + 1) *
                                            sizeof(uint64_t)));
     g->deg_prefix_version = ~0ull;
   }
