@@ -928,16 +928,16 @@ def main():
     # algorithmic bytes: the row-merge model of the whole insert of the batch
     # (8B + 4 sum(d_old + d_new) + 16|T|), attributed to its dominant
     # kernel, which carries the merge of nearly every touched row; the
-    # tile-input count (4 B in + 4 B out per element the LDS tiles merge)
+    # merge-input count (4 B in + 4 B out per element merged in place)
     # beside it
     achieved = op_bytes / (ms_per * 1e-3) / 1e9 if ms_per > 0 else 0.0
     tile_bytes = 8 * stats["tile_inputs"]
     traffic, traffic_src = None, None
-    tfile = os.path.join(ROOT, "profiles", "k_merge_tile_scale24_batch1e7.traffic.json")
+    tfile = os.path.join(ROOT, "profiles", "k_merge_rows_scale24_batch1e7.traffic.json")
     if os.path.exists(tfile) and args.scale == 24 and B == 10_000_000:
         traffic = json.load(open(tfile)).get("bytes_per_launch")
         traffic_src = ("rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE of this command, "
-                       "profiles/k_merge_tile_scale24_batch1e7.traffic.json")
+                       "profiles/k_merge_rows_scale24_batch1e7.traffic.json")
     roofline = dict(kernel=dom_name, bound="hbm", achieved=achieved,
                     peak=HBM_PEAK_GBS, unit="GB/s", frac=achieved / HBM_PEAK_GBS,
                     traffic=traffic, traffic_source=traffic_src,

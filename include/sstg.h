@@ -120,7 +120,7 @@ typedef struct sstg_update_stats {
   uint64_t batch;          /* pairs passed in */
   uint64_t effective;      /* pairs that changed the graph */
   uint64_t rows;           /* rows touched */
-  uint64_t tile_rows;      /* rows merged in place through LDS */
+  uint64_t tile_rows;      /* rows merged in place, wave by wave */
   uint64_t tile_inputs;    /* their merge inputs (moved suffix + batch run) */
   uint64_t big_rows;       /* rows merged over the flat index space */
   uint64_t staged;         /* elements copied to scratch for big rows */

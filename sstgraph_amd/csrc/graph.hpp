@@ -208,12 +208,6 @@ enum : int {
   kWsTileIdx = 85,
   kWsBigStage = 86,
   kWsBigWork = 87,
-  kWsTileLen = 88,
-  kWsTileSrc = 89,
-  kWsTileDst = 90,
-  kWsTileAlen = 91,
-  kWsTileBst = 92,
-  kWsTileBlk = 93,
   kWsMulti = 94,  // 94..97
   kWsTcDag = 98,
   kWsTcDplus = 99,

@@ -22,9 +22,10 @@
 //                the row's batch run into the row slot (or its new slot);
 //                remove: compact the staged suffix minus the batch run
 //  10. finalize  deg / off / cap of the touched rows
-// Steps 8 and 9 run over a flat index space (one thread per 8 outputs), so a
-// hub row with a million neighbours and a thousand one-edge rows are balanced
-// the same way.
+// Rows of at most kTileMax merge inputs skip steps 8 and 9: k_merge_rows
+// merges them in place, wave by wave.  Steps 8 and 9 run the longer rows over
+// a flat index space (one thread per 8 outputs), so a hub row with a million
+// neighbours is spread over many blocks.
 #include <atomic>
 #include <chrono>
 #include <cstring>
@@ -50,20 +51,16 @@ enum {
   kCtrGarbage = 6,  // elements in slots abandoned by relocation
   kCtrScratch = 7,
   kCtrBig = 12,     // big rows
-  kCtrTile = 13,    // elements (inputs) merged by the LDS tile kernel
+  kCtrTile = 13,    // elements (inputs) of the tile rows
   kCtrTiles = 14,   // tile rows
   kCtrCount = 16,
 };
 
-// Rows whose merge inputs (suffix + batch run) fit in kTileMax elements are
-// merged in place by one block through LDS; larger rows are staged.  A block
-// owns the rows whose inputs start in its kTile range, so its tile holds at
-// most kTile + kTileMax inputs.
 // slots (live elements of capacity) below which removal never compacts
 constexpr uint64_t kShrinkMinElems = 1ull << 20;
-constexpr int kTile = 1536;
+// rows of at most so many merge inputs (moved part and batch run) are merged
+// by one wave each, longer ones flat over all of their outputs
 constexpr int kTileMax = 1536;
-constexpr int kTileLds = kTile + kTileMax;
 
 __device__ __forceinline__ uint64_t grow_cap(uint64_t d, uint32_t n_cols) {
   return slot_capacity(d, n_cols);
@@ -114,7 +111,7 @@ __global__ void k_heads(const uint64_t *B, const uint64_t *ctr, uint64_t nmax,
 
 // One thread per touched row (s < t); slot t gets zero lengths, which the
 // scans read as the end of the rows.  Each row is classed as a tile row
-// (merge inputs <= kTileMax, merged in place through LDS) or a big row
+// (merge inputs <= kTileMax, merged in place by k_merge_rows) or a big row
 // (suffix staged, merged over a flat index space).  p0 is the row position
 // k_mark found for the row's first kept key.
 __global__ void k_segprep(const uint64_t *B, const uint32_t *B_pos,
@@ -186,8 +183,8 @@ __global__ void k_segprep(const uint64_t *B, const uint32_t *B_pos,
 // allocated, big rows, tile rows, and the staged elements and merge work of
 // big rows and the inputs of tile rows.  The same pass compacts the two
 // classes: big row k gets big_idx[k] = its segment and its stage and work
-// offsets; tile row k gets tile_idx[k] and its input offset; each offset
-// array ends with its total (entry nb or nt).  Each block of a fixed grid
+// offsets, tile row k gets tile_idx[k]; the offset arrays end with their
+// totals (entry nb).  Each block of a fixed grid
 // (at most kSegBlocks) owns a contiguous range of slots: a reduce writes its
 // six partials, one block scans them, and each block then scans its range.
 constexpr int kSegSums = 6;
@@ -204,7 +201,7 @@ struct SegScan {
   uint64_t n, per;     // slots (nseg + 1), slots per block
   uint64_t *partials;  // kSegSums x blocks, sum-major; null: one block
   uint32_t blocks;
-  uint64_t *big_idx, *big_stage, *big_work, *tile_idx, *tile_len;
+  uint64_t *big_idx, *big_stage, *big_work, *tile_idx;
   uint64_t *ctr;
   uint64_t *hctr;  // mapped host copy of the counter block, or null
   uint64_t seq;    // written to hctr[kHostFlag] after the counters
@@ -359,7 +356,6 @@ __global__ void __launch_bounds__(kT) k_seg_scan(SegScan a) {
         }
         if (v[j][2]) {
           a.tile_idx[ex[2]] = i;
-          a.tile_len[ex[2]] = ex[5];
         }
       }
 #pragma unroll
@@ -375,7 +371,6 @@ __global__ void __launch_bounds__(kT) k_seg_scan(SegScan a) {
     a.ctr[kCtrTile] = carry[5];
     a.big_stage[carry[1]] = carry[3];
     a.big_work[carry[1]] = carry[4];
-    a.tile_len[carry[2]] = carry[5];
     // the whole block, earlier launches' counters included, for the host
     if (a.hctr) {
       for (int k = 0; k < kCtrCount; k++) a.hctr[k] = a.ctr[k];
@@ -400,9 +395,8 @@ struct SegArgs {
   const uint64_t *stage_off;
   const uint64_t *work_off;
   uint64_t nb;
-  // tile rows, compacted: segment ids and exclusive input offsets
+  // tile rows, compacted: segment ids
   const uint64_t *tile_idx;
-  const uint64_t *tile_off;
   uint64_t nt;
 };
 
@@ -621,223 +615,216 @@ __global__ void __launch_bounds__(kT)
   }
 }
 
-// In-place merge of tile rows through LDS.  Block b owns the tile rows whose
-// input range starts in [b*kTile, (b+1)*kTile); it loads every input of those
-// rows (old suffix or whole old row, then the batch run) into LDS,
-// synchronises, and only then writes, so a row is never read after it has
-// been overwritten.  Old element x (index j) lands at j + |{batch < x}|
-// (insert), or at j - |{batch < x}| unless it is in the batch (remove);
-// batch element y (index jb, insert) lands at jb + |{old < y}|.
-// Row description of one tile row: where its inputs come from and where its
-// output goes.
-__device__ __forceinline__ void tile_row_info(const SegArgs &a,
-                                              const DevGraph &g, uint64_t i,
-                                              int insert, uint64_t *src,
-                                              uint64_t *dst, uint32_t *alen,
-                                              uint32_t *bstart) {
-  uint64_t s = a.tile_idx[i];
-  uint32_t v = a.seg_v[s];
-  *bstart = (uint32_t)a.seg_idx[s];
-  if (insert && a.alloc_off[s + 1] > a.alloc_off[s]) {  // relocated
-    *src = g.off[v];
-    *alen = a.seg_olddeg[s];
-    *dst = a.pool_tail + a.alloc_off[s];
-  } else {
-    uint32_t p0 = a.seg_p0[s];
-    *src = g.off[v] + p0;
-    *alen = a.seg_olddeg[s] - p0;
-    *dst = g.off[v] + p0;
-  }
-}
+// ---- row merge
+// Where a row's batch keys go is known from the mark step (each kept key's
+// place in the old row), so no id is compared here.  Of the outputs of a row
+// (moved part and keys together), key i is at its place plus i, and every
+// other output is the moved id that many keys before it: a bitmap of the key
+// outputs holds the whole merge, and a popcount below a position is a rank.
+// On remove the bitmap is over the moved part, and an id that stays moves back
+// by the bits before it.
+//
+// A wave takes up to 64 rows, as many at a time as have kRowWindow outputs
+// together, lays them end to end in one flat space with a second bitmap of the
+// row starts, and walks it 64 positions at a time: two mask ranks give a
+// position its row and its key count, and one load from either the old row or
+// the batch is its value.  Lanes stay full whatever the rows' lengths.  Pieces
+// go from the back on insert and from the front on remove, in groups, each
+// loaded before the one in front of it is stored, so a row is merged in place
+// with no staging: what a piece overwrites has been read.
+//
+// A wave's rows are in runs of kRowRun consecutive ones, the runs a stride of
+// all waves apart: the long rows of a skewed graph are neighbours, and as many
+// of them in one wave held the launch up (64 consecutive rows: 0.3 ms more for
+// the 1e7-edge batch).  Each lane first walks the chain of descriptors of one
+// row (segment, vertex, slot), so a wave pays those round trips once.
+//
+// Bound by the latency of its loads (waves wait three quarters of their
+// cycles; 2.5 GB of traffic at 3.8 TB/s).  1e7-edge insert at rMat scale 24, 3.34M rows,
+// 220M outputs: 0.66 ms, where inputs staged in LDS and ranked by binary
+// searches among the other side's values took 0.87 and 0.09 for descriptors
+// and degrees; a wave per row with the keys as scalars took 1.0-1.6.
+constexpr int kRowT = 256;
+constexpr int kRowWaves = kRowT / kWave;
+constexpr uint32_t kRowWindow = 4096;    // flat positions at a time
+constexpr int kRowsAhead = 4;            // pieces of 64 per group of loads
+constexpr uint32_t kRowLane = 8;         // keys up to which a lane sets its row's
+constexpr uint64_t kRowSpread = 16384;   // waves wanted
+constexpr uint32_t kRowRun = 4;          // consecutive rows of a wave
+static_assert(kTileMax <= (int)kRowWindow, "a row fits a window");
+static_assert(kRowWindow == 64 * kWave, "a lane per 64 positions");
 
-constexpr int kTileRows = 128;  // rows per block described in LDS
-static_assert(kTileRows <= 256, "tile rows are numbered in bytes");
-// k_merge_tile runs 256 threads over one LDS tile: the 12 KB tile, a
-// 128-row table and the 3 KB row map take 18.5 KB, so eight tiles (the wave
-// limit) are in flight per CU; tiles with more rows read their row
-// descriptors from HBM and search them.  The block shape was chosen by
-// timing the 1e7-edge insert at scale 24, before the input loads were
-// issued together (input range / longest tile row:
-// 1536 / 1536 merge 1.046 ms, insert 2.50 ms; 1024 / 2048 1.09 / 2.54;
-// 2048 / 1024 1.015 / 2.66 and 1792 / 1280 1.01 / 2.60, whose longer rows
-// go to the slower big-row path; 2048 / 1536 1.09 / 2.54 and 1536 / 2048
-// 1.08 / 2.53 with a 14 KB tile, seven tiles per CU; 1.40 ms with
-// 1024-thread blocks).
-constexpr int kMergeThreads = 256;
-constexpr int kMergeItems = kTileLds / kMergeThreads;
-
-// Flat descriptors of the tile rows (written after any pool rebuild, so the
-// row offsets they hold are current): input source, output destination,
-// old-part length and start of the batch run.
-__global__ void k_tile_rows(SegArgs a, DevGraph g, int insert,
-                            uint64_t *t_src, uint64_t *t_dst,
-                            uint32_t *t_alen, uint32_t *t_bst) {
-  uint64_t i = (uint64_t)blockIdx.x * kT + threadIdx.x;
-  if (i >= a.nt) return;
-  uint64_t src, dst;
-  uint32_t alen, bst;
-  tile_row_info(a, g, i, insert, &src, &dst, &alen, &bst);
-  t_src[i] = src;
-  t_dst[i] = dst;
-  t_alen[i] = alen;
-  t_bst[i] = bst;
-}
-
-// First tile row of each block and that row's input offset, side by side:
-// blk[2b] = r0 = lower_bound(tile_off, b*kTile), blk[2b+1] = tile_off[r0].
-// A merge block reads its range and the next one's in one 32-byte load
-// instead of two dependent ones.
-__global__ void k_tile_blocks(const uint64_t *tile_off, uint64_t nt,
-                              uint64_t nblocks, uint64_t *blk) {
-  uint64_t b = (uint64_t)blockIdx.x * kT + threadIdx.x;
-  if (b > nblocks) return;
-  const uint64_t r0 =
-      b == nblocks ? nt : lower_bound_dev(tile_off, nt, b * (uint64_t)kTile);
-  blk[2 * b] = r0;
-  blk[2 * b + 1] = tile_off[r0];
-}
-
-__global__ void __launch_bounds__(kMergeThreads)
-    k_merge_tile(SegArgs a, DevGraph g, int insert, const uint64_t *blk,
-                 const uint64_t *t_src, const uint64_t *t_dst,
-                 const uint32_t *t_alen, const uint32_t *t_bst) {
-  __shared__ uint32_t buf[kTileLds];
-  __shared__ uint32_t rstart[kTileRows + 1];  // input offset relative to e0
-  __shared__ uint32_t ralen[kTileRows];
-  __shared__ uint32_t rbstart[kTileRows];
-  __shared__ uint64_t rsrc[kTileRows];
-  __shared__ uint64_t rdst[kTileRows];
-  __shared__ uint8_t rmap[kTileLds];  // tile row of each input (table path)
-  const uint64_t *bk = blk + 2 * (uint64_t)blockIdx.x;
-  const uint64_t r0 = bk[0], e0 = bk[1], r1 = bk[2], e1 = bk[3];
-  if (r0 >= r1) return;
-  const uint32_t W = (uint32_t)(e1 - e0);
-  const uint32_t nrows = (uint32_t)(r1 - r0);
-  const bool table = nrows <= (uint32_t)kTileRows;
-  if (table) {
-    for (uint32_t r = threadIdx.x; r < nrows; r += kMergeThreads) {
-      rstart[r] = (uint32_t)(a.tile_off[r0 + r] - e0);
-      ralen[r] = t_alen[r0 + r];
-      rbstart[r] = t_bst[r0 + r];
-      rsrc[r] = t_src[r0 + r];
-      rdst[r] = t_dst[r0 + r];
-    }
-    if (threadIdx.x == 0) rstart[nrows] = W;
-    __syncthreads();
-    // each wave paints whole rows into the row map (coalesced LDS bytes), so
-    // that an input finds its row with one read instead of a search
-    const uint32_t ln = threadIdx.x % kWave;
-    for (uint32_t r = threadIdx.x / kWave; r < nrows;
-         r += kMergeThreads / kWave) {
-      const uint32_t b1 = rstart[r + 1];
-      for (uint32_t e = rstart[r] + ln; e < b1; e += kWave) rmap[e] = (uint8_t)r;
-    }
-    __syncthreads();
-  }
-  // Every input's address first, then all of a thread's loads, then their
-  // LDS stores: a thread keeps up to kMergeItems loads in flight (with one
-  // store after each load, the compiler waited for every load in turn).  A
-  // batch input is the low word of its 64-bit key.  Slots past the tile
-  // load the pool's first word (always there when tile rows exist) and are
-  // not stored, so the loads need no branch.
-  uint16_t row_of[kMergeItems];
-  const uint32_t *ptr[kMergeItems];
-  const uint32_t *bw = reinterpret_cast<const uint32_t *>(a.B);
-  if (table) {
+template <bool INSERT>
+__global__ void __launch_bounds__(kRowT)
+    k_merge_rows(SegArgs a, const uint32_t *B_pos, DevGraph g, uint32_t per) {
+  __shared__ uint32_t kbits[kRowWaves][kRowWindow / 32];
+  __shared__ uint32_t rbits[kRowWaves][kRowWindow / 32];
+  __shared__ uint64_t lsrc[kRowWaves][kWave], ldst[kRowWaves][kWave];
+  __shared__ uint32_t lkey[kRowWaves][kWave];
+  const uint32_t lane = lane_id(), w = threadIdx.x / kWave;
+  const uint32_t *blo = reinterpret_cast<const uint32_t *>(a.B);
+  const uint64_t wave = (uint64_t)blockIdx.x * kRowWaves + w;
+  const uint64_t waves = (uint64_t)gridDim.x * kRowWaves;
+  const uint64_t mine =
+      ((uint64_t)(lane / kRowRun) * waves + wave) * kRowRun + lane % kRowRun;
+  const bool have = lane < per && mine < a.nt;  // a prefix of the lanes
+  const uint32_t nrows = (uint32_t)__popcll(__ballot(have));
+  if (nrows == 0) return;  // whole waves (no block barrier below)
+  const uint64_t s = a.tile_idx[have ? mine : 0];
+  const uint32_t bs = (uint32_t)a.seg_idx[s];
+  const uint32_t be = (uint32_t)(s + 1 < a.t ? a.seg_idx[s + 1] : a.b);
+  const uint32_t v = a.seg_v[s], od = a.seg_olddeg[s], p0 = a.seg_p0[s];
+  const uint64_t al = a.alloc_off[s], al1 = a.alloc_off[s + 1];
+  const uint64_t ro = g.off[v];
+  const bool moved = INSERT && al1 > al;  // to a fresh slot, all of it
+  const uint32_t q0 = moved ? 0u : p0;
+  const uint64_t src = ro + q0, dst = moved ? a.pool_tail + al : ro + p0;
+  const uint32_t alen = od - q0, blen = be - bs;
+  const uint32_t len = have ? (INSERT ? alen + blen : alen) : 0u;
+  const uint32_t end = wave_inclusive_sum(len);  // flat, over all of the rows
+  const uint32_t kend = wave_inclusive_sum(have ? blen : 0u);
+  uint32_t *kb = kbits[w], *rb = rbits[w];
+  for (uint32_t l0 = 0; l0 < nrows;) {  // uniform
+    // the rows of this window: [l0, l1)
+    const uint32_t base =
+        l0 ? (uint32_t)__builtin_amdgcn_readlane(end, l0 - 1) : 0u;
+    const uint32_t kbase =
+        l0 ? (uint32_t)__builtin_amdgcn_readlane(kend, l0 - 1) : 0u;
+    const bool in = have && lane >= l0 && end - base <= kRowWindow;
+    const uint32_t l1 = l0 + (uint32_t)__popcll(__ballot(in));
+    const uint32_t total =
+        (uint32_t)__builtin_amdgcn_readlane(end, l1 - 1) - base;
+    const uint32_t start = end - len - base;
+    const uint32_t kb0 = kend - blen - kbase;  // keys of the rows before
 #pragma unroll
-    for (int k = 0; k < kMergeItems; k++) {
-      const uint32_t e = threadIdx.x + (uint32_t)k * kMergeThreads;
-      row_of[k] = 0;
-      ptr[k] = g.pool;
-      if (e < W) {
-        const uint32_t r = rmap[e];
-        const uint32_t alen = ralen[r], j = e - rstart[r];
-        row_of[k] = (uint16_t)r;
-        ptr[k] = j < alen ? g.pool + rsrc[r] + j
-                          : bw + 2 * ((uint64_t)rbstart[r] + (j - alen));
+    for (uint32_t i = 0; i < kRowWindow / 32; i += kWave) {
+      kb[i + lane] = 0;
+      rb[i + lane] = 0;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    if (in) {
+      // a bit before each row but the first, so that the bits below a
+      // position are the rows that start at or before it
+      if (start) atomicOr(&rb[(start - 1) >> 5], 1u << ((start - 1) & 31));
+      lsrc[w][lane] = src - start + (INSERT ? kb0 : 0u);
+      ldst[w][lane] = dst - start + (INSERT ? 0u : kb0);
+      lkey[w][lane] = bs - kb0;
+    }
+    // the key bits: short runs by the row's lane, long ones by the wave
+    const uint32_t from = start - q0;  // wraps; from + place is exact
+    if (in && blen <= kRowLane) {
+      uint32_t pos[kRowLane];
+#pragma unroll
+      for (uint32_t i = 0; i < kRowLane; i++)
+        pos[i] = B_pos[bs + (i < blen ? i : 0u)];
+#pragma unroll
+      for (uint32_t i = 0; i < kRowLane; i++)
+        if (i < blen) {
+          const uint32_t o = from + pos[i] + (INSERT ? i : 0u);
+          atomicOr(&kb[o >> 5], 1u << (o & 31));
+        }
+    }
+    uint64_t many = __ballot(in && blen > kRowLane);
+    while (many) {  // uniform
+      const uint32_t l = (uint32_t)__ffsll((unsigned long long)many) - 1;
+      many &= many - 1;
+      const uint32_t b = __builtin_amdgcn_readlane(bs, l);
+      const uint32_t n = __builtin_amdgcn_readlane(blen, l);
+      const uint32_t f = __builtin_amdgcn_readlane(from, l);
+      for (uint32_t i = lane; i < n; i += kWave) {
+        const uint32_t o = f + B_pos[b + i] + (INSERT ? i : 0u);
+        atomicOr(&kb[o >> 5], 1u << (o & 31));
       }
     }
-  } else {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    // lane p holds piece p's masks and the bits before it
+    const uint32_t k0 = kb[2 * lane], k1 = kb[2 * lane + 1];
+    const uint32_t m0 = rb[2 * lane], m1 = rb[2 * lane + 1];
+    const uint32_t kc = (uint32_t)(__popc(k0) + __popc(k1));
+    const uint32_t rc = (uint32_t)(__popc(m0) + __popc(m1));
+    const uint32_t kbef = wave_inclusive_sum(kc) - kc;
+    const uint32_t rbef = wave_inclusive_sum(rc) - rc;
+    const uint32_t pieces = (total + kWave - 1) / kWave;
+    struct Group {
+      uint32_t x[kRowsAhead];
+      bool keep[kRowsAhead];
+      uint64_t to[kRowsAhead];
+    };
+    auto load = [&](uint32_t q, Group &gr) {
+      uint32_t(&x)[kRowsAhead] = gr.x;
+      bool(&keep)[kRowsAhead] = gr.keep;
+      uint64_t(&to)[kRowsAhead] = gr.to;
 #pragma unroll
-    for (int k = 0; k < kMergeItems; k++) {
-      const uint32_t e = threadIdx.x + (uint32_t)k * kMergeThreads;
-      row_of[k] = 0;
-      ptr[k] = g.pool;
-      if (e < W) {
-        const uint64_t i = find_in(a.tile_off, r0, r1 - 1, e0 + e);
-        uint64_t src, dst;
-        uint32_t alen, bst;
-        tile_row_info(a, g, i, insert, &src, &dst, &alen, &bst);
-        const uint32_t j = (uint32_t)(e0 + e - a.tile_off[i]);
-        row_of[k] = (uint16_t)(i - r0);
-        ptr[k] = j < alen ? g.pool + src + j : bw + 2 * ((uint64_t)bst + (j - alen));
+      for (int u = 0; u < kRowsAhead; u++) {
+        const uint32_t qq = q + u < pieces ? q + u : pieces - 1;
+        const uint32_t p = INSERT ? pieces - 1 - qq : qq;
+        const uint32_t ka = __builtin_amdgcn_readlane(k0, p);
+        const uint32_t kz = __builtin_amdgcn_readlane(k1, p);
+        const uint32_t ra = __builtin_amdgcn_readlane(m0, p);
+        const uint32_t rz = __builtin_amdgcn_readlane(m1, p);
+        const uint32_t o = p * kWave + lane;
+        const uint32_t c = __builtin_amdgcn_mbcnt_hi(
+            kz, __builtin_amdgcn_mbcnt_lo(
+                    ka, __builtin_amdgcn_readlane(kbef, p)));
+        const uint32_t row =
+            __builtin_amdgcn_mbcnt_hi(
+                rz, __builtin_amdgcn_mbcnt_lo(
+                        ra, __builtin_amdgcn_readlane(rbef, p))) +
+            l0;
+        const bool key = (((uint64_t)kz << 32 | ka) >> lane) & 1u;
+        const bool ok = o < total && q + u < pieces;
+        // lanes past the end read their row's first input and drop it
+        const uint32_t step = ok ? (INSERT ? o - c : o) : 0u;
+        const uint64_t ls = lsrc[w][row], ld = ldst[w][row];
+        if (INSERT) {
+          const uint32_t *pk = blo + 2 * (uint64_t)(lkey[w][row] + c);
+          const uint32_t *pr = g.pool + (ls + step);
+          const uint32_t *pp = key || !ok ? (ok ? pk : blo) : pr;
+          x[u] = *(const __attribute__((address_space(1))) uint32_t *)pp;
+          keep[u] = ok;
+          to[u] = ld + o;
+        } else {
+          const uint32_t *pp = ok ? g.pool + (ls + step) : blo;
+          x[u] = *(const __attribute__((address_space(1))) uint32_t *)pp;
+          keep[u] = ok && !key;
+          to[u] = ld + o - c;
+        }
       }
+    };
+    auto store = [&](const Group &gr) {
+#pragma unroll
+      for (int u = 0; u < kRowsAhead; u++)
+        if (gr.keep[u]) g.pool[gr.to[u]] = gr.x[u];
+    };
+    // a group is loaded before the one in front of it is stored: neither
+    // order of the two touches what the other reads
+    Group ga, gb;
+    load(0, ga);
+    for (uint32_t q = 0; q < pieces; q += 2 * kRowsAhead) {  // uniform
+      load(q + kRowsAhead, gb);
+      __builtin_amdgcn_sched_barrier(0);
+      store(ga);
+      load(q + 2 * kRowsAhead, ga);
+      __builtin_amdgcn_sched_barrier(0);
+      store(gb);
     }
+    l0 = l1;
   }
-  uint32_t val[kMergeItems];
-#pragma unroll
-  for (int k = 0; k < kMergeItems; k++)  // device memory: global, not flat, loads
-    val[k] = *(const __attribute__((address_space(1))) uint32_t *)ptr[k];
-#pragma unroll
-  for (int k = 0; k < kMergeItems; k++) {
-    const uint32_t e = threadIdx.x + (uint32_t)k * kMergeThreads;
-    if (e < W) buf[e] = val[k];
-  }
-  __syncthreads();
-#pragma unroll
-  for (int k = 0; k < kMergeItems; k++) {
-    const uint32_t e = threadIdx.x + (uint32_t)k * kMergeThreads;
-    if (e >= W) continue;
-    const uint32_t r = row_of[k];
-    uint32_t base, alen, blen;
-    uint64_t dst;
-    if (table) {
-      base = rstart[r];
-      blen = rstart[r + 1] - base - ralen[r];
-      alen = ralen[r];
-      dst = rdst[r];
-    } else {
-      uint64_t i = r0 + r;
-      uint64_t src;
-      uint32_t bst;
-      tile_row_info(a, g, i, insert, &src, &dst, &alen, &bst);
-      base = (uint32_t)(a.tile_off[i] - e0);
-      blen = (uint32_t)(a.tile_off[i + 1] - a.tile_off[i]) - alen;
-    }
-    const uint32_t j = e - base;
-    const uint32_t *la = buf + base, *lb = buf + base + alen;
-    const uint32_t x = buf[e];
-    uint32_t *out = g.pool + dst;
-    if (j < alen) {
-      uint32_t l = 0, h = blen;  // batch elements below x
-      while (l < h) {
-        uint32_t m = (l + h) >> 1;
-        if (lb[m] < x)
-          l = m + 1;
-        else
-          h = m;
-      }
-      if (insert)
-        out[j + l] = x;
-      else if (!(l < blen && lb[l] == x))
-        out[j - l] = x;
-    } else if (insert) {
-      uint32_t l = 0, h = alen;  // old elements below x
-      while (l < h) {
-        uint32_t m = (l + h) >> 1;
-        if (la[m] < x)
-          l = m + 1;
-        else
-          h = m;
-      }
-      out[(j - alen) + l] = x;
+  if (have) {
+    g.deg[v] = INSERT ? od + blen : od - blen;
+    if (moved) {
+      g.off[v] = dst;
+      g.cap[v] = (uint32_t)(al1 - al);
     }
   }
 }
 
+// deg, off and cap of the big rows
 __global__ void k_finalize(SegArgs a, DevGraph g, int insert) {
-  uint64_t s = (uint64_t)blockIdx.x * kT + threadIdx.x;
-  if (s >= a.t) return;
+  const uint64_t i = (uint64_t)blockIdx.x * kT + threadIdx.x;
+  if (i >= a.nb) return;
+  const uint64_t s = a.big_idx[i];
   uint64_t bs = a.seg_idx[s], be = (s + 1 < a.t) ? a.seg_idx[s + 1] : a.b;
   uint32_t blen = (uint32_t)(be - bs);
   uint32_t v = a.seg_v[s];
@@ -1191,8 +1178,7 @@ static int update_chunk(sstg_graph *g, const uint32_t *src, const uint32_t *dst,
   uint32_t *seg_v = nullptr, *seg_p0 = nullptr, *seg_od = nullptr,
            *seg_stage = nullptr, *seg_tile = nullptr;
   uint64_t *seg_alloc = nullptr, *seg_work = nullptr, *big_idx = nullptr,
-           *tile_idx = nullptr, *big_stage = nullptr, *big_work = nullptr,
-           *tile_len = nullptr;
+           *tile_idx = nullptr, *big_stage = nullptr, *big_work = nullptr;
   uint8_t *is_big = nullptr, *is_tile = nullptr;
   SSTG_TRY(ws.get(kWsSegV, nseg + 1, &seg_v));
   SSTG_TRY(ws.get(kWsSegP0, nseg + 1, &seg_p0));
@@ -1207,7 +1193,6 @@ static int update_chunk(sstg_graph *g, const uint32_t *src, const uint32_t *dst,
   SSTG_TRY(ws.get(kWsTileIdx, nseg + 1, &tile_idx));
   SSTG_TRY(ws.get(kWsBigStage, nseg + 1, &big_stage));
   SSTG_TRY(ws.get(kWsBigWork, nseg + 1, &big_work));
-  SSTG_TRY(ws.get(kWsTileLen, nseg + 1, &tile_len));
   SSTG_LAUNCH(k_segprep, blocks(nseg + 1), kT, 0, s, (const uint64_t *)B,
               (const uint32_t *)B_pos, (const uint64_t *)ctr, (const uint64_t *)seg_idx, g->view(),
               insert ? 1 : 0, g->n_cols, nseg, seg_v, seg_p0, seg_od,
@@ -1226,7 +1211,6 @@ static int update_chunk(sstg_graph *g, const uint32_t *src, const uint32_t *dst,
     sc.big_stage = big_stage;
     sc.big_work = big_work;
     sc.tile_idx = tile_idx;
-    sc.tile_len = tile_len;
     sc.ctr = ctr;
     sc.hctr = g->host_ctr_dev;
     sc.seq = ++g->host_seq;
@@ -1293,26 +1277,19 @@ static int update_chunk(sstg_graph *g, const uint32_t *src, const uint32_t *dst,
   a.work_off = big_work;
   a.nb = nb;
   a.tile_idx = tile_idx;
-  a.tile_off = tile_len;
   a.nt = nt;
-  if (tile_tot) {
-    const uint64_t nblk = ceil_div(tile_tot, kTile);
-    uint64_t *t_src = nullptr, *t_dst = nullptr, *blk = nullptr;
-    uint32_t *t_alen = nullptr, *t_bst = nullptr;
-    SSTG_TRY(ws.get(kWsTileSrc, nt + 1, &t_src));
-    SSTG_TRY(ws.get(kWsTileDst, nt + 1, &t_dst));
-    SSTG_TRY(ws.get(kWsTileAlen, nt + 1, &t_alen));
-    SSTG_TRY(ws.get(kWsTileBst, nt + 1, &t_bst));
-    SSTG_TRY(ws.get(kWsTileBlk, 2 * (nblk + 1), &blk));
-    SSTG_LAUNCH(k_tile_rows, blocks(nt), kT, 0, s, a, g->view(),
-                insert ? 1 : 0, t_src, t_dst, t_alen, t_bst);
-    SSTG_LAUNCH(k_tile_blocks, blocks(nblk + 1), kT, 0, s,
-                (const uint64_t *)tile_len, nt, nblk, blk);
-    SSTG_LAUNCH(k_merge_tile, nblk, kMergeThreads, 0, s, a, g->view(),
-                insert ? 1 : 0,
-                (const uint64_t *)blk, (const uint64_t *)t_src,
-                (const uint64_t *)t_dst, (const uint32_t *)t_alen,
-                (const uint32_t *)t_bst);
+  if (nt) {
+    // enough waves to fill the chip, and up to 64 rows each
+    const uint64_t want = ceil_div(nt, kRowSpread);
+    const uint32_t per = (uint32_t)(
+        want >= kWave ? kWave : ceil_div(want, kRowRun) * kRowRun);
+    const uint64_t nblk = ceil_div(ceil_div(nt, (uint64_t)per), kRowWaves);
+    if (insert)
+      SSTG_LAUNCH(k_merge_rows<true>, nblk, kRowT, 0, s, a,
+                  (const uint32_t *)B_pos, g->view(), per);
+    else
+      SSTG_LAUNCH(k_merge_rows<false>, nblk, kRowT, 0, s, a,
+                  (const uint32_t *)B_pos, g->view(), per);
   }
   if (stage_tot)
     SSTG_LAUNCH(k_stage, chunk_blocks(stage_tot), kT, 0, s, a, g->view(),
@@ -1325,7 +1302,8 @@ static int update_chunk(sstg_graph *g, const uint32_t *src, const uint32_t *dst,
       SSTG_LAUNCH(k_compact_remove, chunk_blocks(work_tot), kT, 0, s, a,
                   g->view(), work_tot);
   }
-  SSTG_LAUNCH(k_finalize, blocks(t), kT, 0, s, a, g->view(), insert ? 1 : 0);
+  if (nb)
+    SSTG_LAUNCH(k_finalize, blocks(nb), kT, 0, s, a, g->view(), insert ? 1 : 0);
   // track symmetry through small batches; a batch that is large next to the
   // graph leaves it unknown (checked in full when a traversal needs it)
   const bool was_symmetric = g->sym_version == g->version && g->symmetric &&
