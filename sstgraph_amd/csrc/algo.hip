@@ -645,19 +645,75 @@ __global__ void k_sigma_push(DevGraph g, const uint32_t *list, uint64_t count,
   }
 }
 
-// Clears *flag if some stored edge (u, v) has no reverse (v, u).
-__global__ void k_symmetry(DevGraph g, const uint64_t *prefix, uint64_t m,
-                           uint32_t *flag) {
-  uint64_t e = ((uint64_t)blockIdx.x * kT + threadIdx.x) * 8;
-  if (e >= m) return;
-  uint64_t end = e + 8 < m ? e + 8 : m;
-  uint64_t u = find_segment(prefix, g.n, e);
-  for (; e < end; e++) {
-    while (e >= prefix[u + 1]) u++;
-    uint32_t v = g.pool[g.off[u] + (e - prefix[u])];
-    bool ok = false;
-    if (v < g.n) ok = row_has(g.pool + g.off[v], g.deg[v], (uint32_t)u);
+// Whether every stored edge (u, v) has its reverse (v, u).  The edges from a
+// vertex to one ranked below it by (degree, id) map to the edges to one ranked
+// above, one to one; if each has its reverse and the two kinds are equally
+// many, every edge has one.  So only the first kind is searched, half of the
+// edges and each in the shorter of the two rows.  Clears *flag at an edge
+// without its reverse; part gets each block's difference of the two kinds.
+// Searching every edge in its other end's row took the first BFS
+// of a rMat scale-24 graph from 15.7 to 33.0 ms, 10.1 at scale 22 against 5.4.
+__global__ void __launch_bounds__(kT)
+    k_symmetry(DevGraph g, const uint64_t *prefix, uint64_t m, uint32_t *flag,
+               int64_t *part) {
+  constexpr int kEdges = 8;
+  __shared__ int64_t wsum[kT / kWave];
+  const uint64_t e0 = ((uint64_t)blockIdx.x * kT + threadIdx.x) * kEdges;
+  int64_t diff = 0;
+  if (e0 < m) {
+    uint64_t u = find_segment(prefix, g.n, e0);
+    uint64_t next = prefix[u + 1], at = g.off[u] - prefix[u];
+    uint32_t du = g.deg[u], us[kEdges], dus[kEdges], v[kEdges], dv[kEdges];
+    uint64_t place[kEdges];
+#pragma unroll
+    for (int j = 0; j < kEdges; j++) {  // past the end: the last edge again
+      const uint64_t e = e0 + j < m ? e0 + j : m - 1;
+      while (e >= next) {
+        u++;
+        at = g.off[u] - next;
+        next = prefix[u + 1];
+        du = g.deg[u];
+      }
+      us[j] = (uint32_t)u;
+      dus[j] = du;
+      place[j] = at + e;
+    }
+#pragma unroll
+    for (int j = 0; j < kEdges; j++) v[j] = g.pool[place[j]];
+#pragma unroll
+    for (int j = 0; j < kEdges; j++) dv[j] = v[j] < g.n ? g.deg[v[j]] : 0u;
+    bool ok = true;
+#pragma unroll
+    for (int j = 0; j < kEdges; j++) {
+      if (e0 + j >= m || v[j] == us[j]) continue;
+      const bool below = dv[j] < dus[j] || (dv[j] == dus[j] && v[j] < us[j]);
+      diff += below ? 1 : -1;
+      if (below)
+        ok = ok && v[j] < g.n && row_has(g.pool + g.off[v[j]], dv[j], us[j]);
+    }
     if (!ok) *flag = 0;
+  }
+  diff = wave_sum(diff);
+  if ((threadIdx.x & (kWave - 1)) == 0) wsum[threadIdx.x / kWave] = diff;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < kT / kWave; w++) diff += wsum[w];
+    part[blockIdx.x] = diff;
+  }
+}
+
+// *flag cleared unless the differences add up to none (one block)
+__global__ void __launch_bounds__(kT)
+    k_symmetry_sum(const int64_t *part, uint64_t nb, uint32_t *flag) {
+  __shared__ int64_t wsum[kT / kWave];
+  int64_t t = 0;
+  for (uint64_t i = threadIdx.x; i < nb; i += kT) t += part[i];
+  t = wave_sum(t);
+  if ((threadIdx.x & (kWave - 1)) == 0) wsum[threadIdx.x / kWave] = t;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < kT / kWave; w++) t += wsum[w];
+    if (t != 0) *flag = 0;
   }
 }
 
@@ -691,8 +747,11 @@ int graph_is_symmetric(sstg_graph *g, bool *out) {
   if (g->m) {
     const uint64_t *prefix = nullptr;
     SSTG_TRY(graph_degree_prefix(g, &prefix));
-    SSTG_LAUNCH(k_symmetry, ceil_div(ceil_div(g->m, 8), kT), kT, 0, s,
-                g->view(), prefix, g->m, flag);
+    const uint64_t nb = ceil_div(ceil_div(g->m, 8), kT);
+    int64_t *part = nullptr;
+    SSTG_TRY(g->ws.get(kWsSym, nb, &part));
+    SSTG_LAUNCH(k_symmetry, nb, kT, 0, s, g->view(), prefix, g->m, flag, part);
+    SSTG_LAUNCH(k_symmetry_sum, 1, kT, 0, s, (const int64_t *)part, nb, flag);
   }
   SSTG_HIP(hipMemcpyAsync(g->host_rb + 20, flag, sizeof(uint32_t),
                           hipMemcpyDeviceToHost, s));

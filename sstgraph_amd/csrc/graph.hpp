@@ -243,6 +243,7 @@ enum : int {
   kWsSmallFound = 149,  // small updates: each pair's row search
   kWsRebuild = 150,     // 150..152 pool rebuild: capacities, offsets, prefix
   kWsPush = 155,        // 155..159 device-driven BFS levels
+  kWsSym = 165,         // symmetry check: per-block partials
   kWsBins = 153,        // 153, 154 graph_bins: block counts, totals
 };
 
