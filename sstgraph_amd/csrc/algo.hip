@@ -707,7 +707,16 @@ __global__ void __launch_bounds__(kT)
     k_symmetry_sum(const int64_t *part, uint64_t nb, uint32_t *flag) {
   __shared__ int64_t wsum[kT / kWave];
   int64_t t = 0;
-  for (uint64_t i = threadIdx.x; i < nb; i += kT) t += part[i];
+  for (uint64_t i = threadIdx.x; i < nb; i += 8 * kT) {
+    int64_t p[8];  // in flight together: 0.28 ms for 185K partials one by one
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+      const uint64_t at = i + (uint64_t)j * kT;
+      p[j] = part[at < nb ? at : i];
+    }
+#pragma unroll
+    for (int j = 0; j < 8; j++) t += i + (uint64_t)j * kT < nb ? p[j] : 0;
+  }
   t = wave_sum(t);
   if ((threadIdx.x & (kWave - 1)) == 0) wsum[threadIdx.x / kWave] = t;
   __syncthreads();

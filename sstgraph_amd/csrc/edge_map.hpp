@@ -89,11 +89,6 @@ constexpr int kT = 256;
 constexpr int kChunk = 8;
 constexpr int kBitmapRounds = 8;  // 512 vertices per wave in k_bits
 
-__global__ void k_clear_u32(uint32_t *p, uint64_t n) {
-  uint64_t i = (uint64_t)blockIdx.x * kT + threadIdx.x;
-  if (i < n) p[i] = 0;
-}
-
 __global__ void k_frontier_degrees(DevGraph g, const uint32_t *q, uint64_t nq,
                                    uint32_t least, uint64_t *out) {
   uint64_t i = (uint64_t)blockIdx.x * kT + threadIdx.x;
