@@ -972,6 +972,7 @@ static int bfs_core(sstg_graph *g, uint32_t src, uint32_t *level,
   ctx.rev = 2 * c[kPushLevels + 2] < c[kPushLevels + 3];
   uint64_t qs = 0, nf = 1, mf = src_deg;
   uint64_t explored = src_deg;  // edges of visited vertices
+  bool mf_of_batch = false;  // mf is a batch's count of the frontier's edges
   bool bottom_up = false;
   bool vis_stale = false;  // bottom-up steps do not maintain the filter
   const double alpha = g->bfs_alpha, beta = g->bfs_beta;
@@ -1035,10 +1036,16 @@ static int bfs_core(sstg_graph *g, uint32_t src, uint32_t *level,
       explored += h[4];
       prev_nf = h[5];
       mf = h[6];
+      mf_of_batch = false;
       bottom_up = false;
       continue;
     }
-    if (batch_done || (!want_bu && mf <= push_cap && nf <= kPushCountMask)) {
+    // What the device compares with the cap counts a vertex without edges as
+    // one edge, which only a graph with one-directional edges reaches; mf
+    // counts it so too after a batch, and is short of it by at most nf else.
+    const uint64_t push_mf = symmetric || mf_of_batch ? mf : mf + nf;
+    if (batch_done ||
+        (!want_bu && push_mf <= push_cap && nf <= kPushCountMask)) {
       if (!batch_done) {
         if (pre_front != queue + qs) {
           // offsets from a bottom-up step's end serve as they are: its
@@ -1056,8 +1063,9 @@ static int bfs_core(sstg_graph *g, uint32_t src, uint32_t *level,
         SSTG_TRY(push_batch(L));
       }
       batch_done = false;
-      int k = 0;
-      while (k < push_steps && nf > 0 && mf <= push_cap) {  // expanded on the device
+      int k = 0;  // levels expanded, by the counters the device went by
+      while (k < push_steps && (c[k] & kPushCountMask) &&
+             (c[k] >> kPushCountBits) <= push_cap) {
         k++;
         qs += nf;
         prev_nf = nf;
@@ -1067,8 +1075,6 @@ static int bfs_core(sstg_graph *g, uint32_t src, uint32_t *level,
         L++;
         if (run) run->level_start.push_back(qs + nf);
       }
-      vis_stale = vis_stale || k > 0;
-      bottom_up = false;
       // after all its steps the last frontier's total is still to be written
       pre_front = k < push_steps ? queue + qs : nullptr;
       pre_cur = cur[k];
@@ -1088,7 +1094,13 @@ static int bfs_core(sstg_graph *g, uint32_t src, uint32_t *level,
                          .count());
         t_level = t1;
       }
-      continue;
+      if (k > 0) {
+        mf_of_batch = true;
+        vis_stale = true;
+        bottom_up = false;
+        continue;
+      }
+      // the frontier given is over the cap: a step sized by the host
     }
     EdgeMapResult res;
     uint32_t *next = queue + qs + nf;
@@ -1121,6 +1133,7 @@ static int bfs_core(sstg_graph *g, uint32_t src, uint32_t *level,
     prev_nf = nf;
     nf = res.count;
     mf = res.degree_sum;  // ~0 after a bottom-up step: not computed
+    mf_of_batch = false;
     if (mf != ~0ull) explored += mf;
     L++;
     if (run) run->level_start.push_back(qs + nf);

@@ -1,12 +1,13 @@
 """BFS where its top-down levels change hands: device-driven batches, the
 one-block tail and host-sized pushes, with frontiers around the tile and cap
-sizes, chains longer than any batch, and vertices without out-edges."""
+sizes, chains longer than any batch, and vertices without out-edges, many of
+them in one frontier."""
 import numpy as np
 import pytest
 
 import sstgraph_amd as S
 from oracle import oracle as O
-from tests.gpu_common import need_gpu, say
+from tests.gpu_common import need_gpu, rel_close, say
 
 pytestmark = pytest.mark.gpu
 EMV = S.EdgeMapVertexMap
@@ -37,6 +38,7 @@ def _check(n, s, d, sources, sym=True):
         keys = keys * np.uint64(n) + cols
         assert np.isin(p.astype(np.uint64) * np.uint64(n) + v.astype(np.uint64),
                        keys).all()
+    return off, cols, g
 
 
 @pytest.mark.parametrize("leaves", [1, 511, 512, 513, 2047, 2049, 131071,
@@ -84,3 +86,43 @@ def test_random_graph_any_source(sym):
     rng = np.random.default_rng(3)
     s, d = rng.integers(0, n, 2 * n), rng.integers(0, n, 2 * n)
     _check(n, s, d, [0, 7, n - 1], sym)
+
+
+CAP = 1 << 20  # most edges of a device-driven frontier in a graph of over 2^22
+
+
+@pytest.mark.parametrize("sinks,edges", [
+    (CAP + CAP // 2, 3000),   # the second frontier itself over the cap
+    (CAP - 3000, 6000),       # degrees 2: sinks and edges 3000 over
+    (CAP - 6000, 6000),       # edges with a sink counted as one: the cap
+    (CAP - 5999, 6000),       # one over
+    (CAP - 9000, 6000),       # vertices and edges together: the cap
+    (CAP - 8999, 6000),       # one over
+])
+def test_directed_frontier_of_sinks(sinks, edges):
+    """A frontier of about a cap's worth of vertices without out-edges, among
+    them edges / 2 that lead on for three more levels, behind frontiers that
+    only a push sized by the host expands."""
+    need_gpu()
+    on, first = edges // 2, CAP + 1
+    src, a = 0, np.arange(1, first + 1)
+    b = first + 1 + np.arange(sinks + on)
+    c = b[-1] + 1 + np.arange(edges)
+    e = c[-1] + 1 + np.arange(5)
+    n = int(e[-1]) + 1 + 4096
+    rng = np.random.default_rng(edges + sinks)
+    lead = rng.permutation(b)[:on]
+    parts = [(np.full(first, src), a), (a[np.arange(len(b)) % first], b),
+             (np.repeat(lead, 2), c), (c[::7], np.full(len(c[::7]), e[0])),
+             (e[:-1], e[1:])]
+    # edges out of reach, up to a graph too large to stay on the device
+    m = sum(len(x) for x, _ in parts)
+    f = n - 4096 + rng.integers(0, 4096, (2, 3 << 20))
+    s = np.concatenate([x for x, _ in parts] + [f[0]]).astype(np.uint32)
+    d = np.concatenate([y for _, y in parts] + [f[1]]).astype(np.uint32)
+    say("sinks", sinks, edges, m)
+    off, cols, g = _check(n, s, d, [src], False)
+    assert len(cols) > 1 << 22 and g.M() == len(cols)
+    assert np.array_equal(EMV.BF(g, src), O.bf(off, cols, src))
+    ok, worst = rel_close(EMV.BC(g, src), O.bc(off, cols, src), 1e-9, 1e-12)
+    assert ok, worst
