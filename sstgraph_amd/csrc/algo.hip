@@ -927,13 +927,12 @@ static int bfs_core(sstg_graph *g, uint32_t src, uint32_t *level,
   ctx.log = log;
   uint32_t *queue = order;
   if (!queue) SSTG_TRY(ws.get(kWsAlgo + 10, (uint64_t)n + 1, &queue));
-  // device-driven levels: alternate frontiers' offsets and rows, of which the
-  // current one's are in pre_cur when it is pre_front
+  // device-driven levels: alternate frontiers' offsets and rows
   const uint64_t push_cap = g->m <= kPushAll ? ~0ull : kPushCap;
   const int push_steps = g->m <= kPushAll ? kPushLevels : kPushLevels / 3;
   const uint64_t pre_n =
       std::min<uint64_t>(n, g->m <= kPushAll ? kPushAll : kPushCap) + 2;
-  PushFront pre_buf[2], pre_cur;
+  PushFront pre_buf[2];
   PushBatch pb;
   for (int i = 0; i < 2; i++) {
     SSTG_TRY(ws.get(kWsPush + i, 2 * pre_n, &pre_buf[i].pre));
@@ -941,18 +940,16 @@ static int bfs_core(sstg_graph *g, uint32_t src, uint32_t *level,
   }
   SSTG_TRY(ws.get(kWsPush + 2, kPushLevels + 1 + 3, &pb.ctr));
   SSTG_TRY(ws.get(kWsPush + 3, kPushLevels + 2, &pb.start));
-  const uint32_t *pre_front = queue;
-  pre_cur = pre_buf[0];
   SSTG_LAUNCH(k_bfs_start, blocks(std::max<uint64_t>(n, ctx.words)), kT, 0, s,
               n, level, parent, src, queue, ctx.vis, ctx.words,
               (const uint32_t *)g->deg, (const uint64_t *)g->off, prefix, pb,
               pre_buf[0], ctx.ctrs, (uint32_t)(2 * em::kStepCtrs));
-  // one batch of push levels from frontier pre_cur (level L), its counters
-  // and the start's three words read back into c
+  // one batch of push levels from frontier first (level L), its counters and
+  // the start's three words read back into c
   PushFront cur[kPushLevels + 1];
   uint64_t c[kPushLevels + 1 + 3];
-  auto push_batch = [&](uint32_t L) -> int {
-    cur[0] = pre_cur;
+  auto push_batch = [&](const PushFront &first, uint32_t L) -> int {
+    cur[0] = first;
     for (int k = 0; k < push_steps; k++) {
       cur[k + 1] = cur[k].pre == pre_buf[0].pre ? pre_buf[1] : pre_buf[0];
       SSTG_LAUNCH(k_push_level, kPushGrid, kPushT, 0, s, g->view(), pb, k,
@@ -966,7 +963,7 @@ static int bfs_core(sstg_graph *g, uint32_t src, uint32_t *level,
   // upper half of the ids and the whole (rows are sorted by id, so when the
   // high ids carry more edges -- as in the reference's rMat, whose hubs have
   // mostly 1 bits -- a frontier vertex is met sooner from a row's end)
-  SSTG_TRY(push_batch(0));
+  SSTG_TRY(push_batch(pre_buf[0], 0));
   bool batch_done = true;
   const uint32_t src_deg = (uint32_t)c[kPushLevels + 1];
   ctx.rev = 2 * c[kPushLevels + 2] < c[kPushLevels + 3];
@@ -1047,20 +1044,19 @@ static int bfs_core(sstg_graph *g, uint32_t src, uint32_t *level,
     if (batch_done ||
         (!want_bu && push_mf <= push_cap && nf <= kPushCountMask)) {
       if (!batch_done) {
-        if (pre_front != queue + qs) {
-          // offsets from a bottom-up step's end serve as they are: its
-          // vertices all have edges
-          if (ctx.fpre_front != queue + qs || ctx.fpre_n != nf || !symmetric)
-            SSTG_TRY(frontier_prefix(g, ctx, queue + qs, nf, nullptr, 1));
-          ctx.fpre_front = nullptr;
-          pre_cur.pre = ctx.fpre;
-          SSTG_TRY(ws.get(kWsPush + 4, nf, &pre_cur.row));
-          SSTG_LAUNCH(k_front_rows, blocks(nf), kT, 0, s, g->view(),
-                      (const uint32_t *)(queue + qs), nf, pre_cur.row);
-        }
+        // offsets from a bottom-up step's end serve as they are: its vertices
+        // all have edges
+        if (ctx.fpre_front != queue + qs || ctx.fpre_n != nf || !symmetric)
+          SSTG_TRY(frontier_prefix(g, ctx, queue + qs, nf, nullptr, 1));
+        ctx.fpre_front = nullptr;
+        PushFront first;
+        first.pre = ctx.fpre;
+        SSTG_TRY(ws.get(kWsPush + 4, nf, &first.row));
+        SSTG_LAUNCH(k_front_rows, blocks(nf), kT, 0, s, g->view(),
+                    (const uint32_t *)(queue + qs), nf, first.row);
         SSTG_LAUNCH(k_push_state, 1, kWave, 0, s, pb, qs, nf,
-                    (const uint64_t *)pre_cur.pre);
-        SSTG_TRY(push_batch(L));
+                    (const uint64_t *)first.pre);
+        SSTG_TRY(push_batch(first, L));
       }
       batch_done = false;
       int k = 0;  // levels expanded, by the counters the device went by
@@ -1075,13 +1071,11 @@ static int bfs_core(sstg_graph *g, uint32_t src, uint32_t *level,
         L++;
         if (run) run->level_start.push_back(qs + nf);
       }
-      // after all its steps the last frontier's total is still to be written
-      pre_front = k < push_steps ? queue + qs : nullptr;
-      pre_cur = cur[k];
       if (k < push_steps && symmetric) {
-        // stopped over the cap: offsets complete for a push (a vertex without
-        // edges, which only a graph with one-directional edges reaches, would
-        // count as one)
+        // stopped over the cap: offsets complete for a push (after all of the
+        // steps their total is still to be written; a vertex without edges,
+        // which only a graph with one-directional edges reaches, would count
+        // as one)
         ctx.fpre = cur[k].pre;
         ctx.fpre_front = queue + qs;
         ctx.fpre_n = nf;
@@ -1104,7 +1098,6 @@ static int bfs_core(sstg_graph *g, uint32_t src, uint32_t *level,
     }
     EdgeMapResult res;
     uint32_t *next = queue + qs + nf;
-    pre_front = nullptr;
     if (want_bu) {
       SSTG_TRY(edge_map_dense(g, ctx, BfsPull{level, parent, L + 1},
                               LevelIs{level, L}, next, &res));
@@ -1337,7 +1330,7 @@ int algo_cc(sstg_graph *g, uint32_t *out) {
   if (g->m && symmetric) {
     uint32_t *samples = nullptr;
     // PageRank's contribution buffer holds the same bytes (8 per vertex)
-  SSTG_TRY(g->ws.get(kWsAlgo + 20, (uint64_t)n * cc::kHookRounds, &samples));
+    SSTG_TRY(g->ws.get(kWsAlgo + 20, (uint64_t)n * cc::kHookRounds, &samples));
     const cc::Slots sl{prefix, nullptr, nullptr, n};
     SSTG_TRY(cc::forest_symmetric(v, sl, p, samples, 1, giant, s));
     SSTG_LAUNCH(k_cc_labels, blocks(n), kT, 0, s, sl, p,
