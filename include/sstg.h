@@ -248,7 +248,8 @@ int sstg_rmat(uint32_t n, uint32_t seed, double a, double b, double c,
  * (continuous batching, flag SSTG_SERVE_COALESCE); queries run concurrently
  * on `slots` slots (own HIP stream and workspace each), admitted in arrival
  * order while a slot is free and their device-memory estimate fits the HBM
- * budget (hbm_budget bytes, 0 = 7/8 of the free memory at creation).  With
+ * budget (hbm_budget bytes, 0 = 7/8 of the free memory at creation); a query
+ * whose estimate is over the whole budget runs alone.  With
  * SSTG_SERVE_SNAPSHOTS an update does not wait for running or queued
  * queries: the graph moves to a device copy of its store and those queries
  * run on the old arrays (held against the budget while they are needed).

@@ -909,6 +909,15 @@ __global__ void __launch_bounds__(kTailThreads)
   }
 }
 
+// bfs_core's buffers, the most of each: queue, frontier and visited bitmaps,
+// frontier offsets, the degree prefix, the bottom-up lists with their degree
+// bins, and the device-driven levels' offsets and rows (two frontiers', and
+// the rows of one that starts a batch).
+uint64_t bfs_bytes(uint64_t n) {
+  const uint64_t push = std::min(n, std::max(kPushAll, kPushCap));
+  return n * 4 + n / 4 + n * 8 + n * 8 + n * (16 + 4) + push * (32 + 8);
+}
+
 // Every level's vertices are appended to the queue (order, or a workspace
 // buffer) whatever the direction, so level L's vertices are
 // queue[level_start[L] .. level_start[L + 1]).  Per level the host reads one
@@ -1315,6 +1324,9 @@ int algo_pagerank_f32k(sstg_graph *g, uint32_t iters, double damping,
 }
 
 // ====================================================================== CC
+// algo_cc's buffers: parents, sampled neighbours, the degree prefix
+uint64_t cc_bytes(uint64_t n) { return n * 4 + n * 4 * cc::kHookRounds + n * 8; }
+
 int algo_cc(sstg_graph *g, uint32_t *out) {
   hipStream_t s = g->stream;
   const uint32_t n = g->n_rows;

@@ -51,6 +51,10 @@ int algo_pagerank_f32k(sstg_graph *g, uint32_t iters, double damping,
 int algo_bc(sstg_graph *g, uint32_t src, double *out);
 int algo_cc(sstg_graph *g, uint32_t *out);
 int algo_tc(sstg_graph *g, uint64_t *out);
+// device bytes BFS and CC take on a graph of n vertices beside the store and
+// their outputs
+uint64_t bfs_bytes(uint64_t n);
+uint64_t cc_bytes(uint64_t n);
 // degree-oriented TC; valid only when every edge has its reverse (tc.hip)
 int tc_oriented(sstg_graph *g, uint64_t *out);
 // sum over u, v in L(u) of |L(u) n L(v)|, L(x) = lists[base[x] .. +len[x])

@@ -23,13 +23,15 @@
 //    own HIP stream, workspace and read-only view of the store), so queries
 //    that arrive while others are on the GPU overlap with them.  They are
 //    admitted in arrival order while a slot is free and their device memory
-//    estimate fits the HBM budget; otherwise they wait.  With
+//    estimate fits the HBM budget; otherwise they wait.  A query whose
+//    estimate is over the whole budget runs alone.  With
 //    SSTG_SERVE_ONE_HEAVY at most one PageRank or TC runs at a time, and
 //    lighter queries admitted behind a waiting one pass it (readers in any
 //    order see the same store).
 //  * With SSTG_SERVE_SNAPSHOTS a query still waiting when an update behind
 //    it could run is pinned to the current store arrays, so the update goes
 //    ahead on a copy and the query later runs on the version it arrived at.
+#include <algorithm>
 #include <atomic>
 #include <chrono>
 #include <condition_variable>
@@ -115,6 +117,7 @@ struct sstg_server {
   std::vector<sstg::StoreSet> spare;     // recycled store arrays
   std::vector<sstg::StoreSet> to_free;   // extra spares for the reaper
   std::thread reaper;
+  bool reaping = false;                  // it is freeing one
   // the update run on the writer thread (one at a time)
   std::thread writer;
   std::vector<sstg::Request *> write_run;
@@ -151,23 +154,36 @@ struct sstg_server {
 namespace sstg {
 namespace {
 
-// Device bytes a query needs beyond the shared store (result + scratch).
-uint64_t estimate(const sstg_graph *g, const sstg_request &r) {
+// Device bytes that a query is refused by if they alone exceed the budget.
+uint64_t least_bytes(const sstg_graph *g, const sstg_request &r) {
   const uint64_t n = g->n_rows;
   switch (r.kind) {
     case SSTG_REQ_BFS:
-      return n * 4 + n * 24;            // levels + queue, flags, bitmaps
+      return n * 4 + n * 24;            // levels + queue, lists
     case SSTG_REQ_PR:
       // ranks, contributions, run ranges; the column-segment layout and its
       // build (4 B per edge + at most one run per edge at 40 B, 1 B per
       // edge of counts) when it applies, else the degree bins
       return n * 32 + (pagerank_segmented_applies(g) ? g->m * 45 : n * 20);
     case SSTG_REQ_CC:
-      return n * 8;
+      return n * 8;                     // labels + parents
     case SSTG_REQ_TC:
       return g->m * 4 + n * 17;         // oriented lists + out-degrees, lists
     default:
       return 0;
+  }
+}
+
+// Device bytes a query takes beyond the shared store (result + scratch): what
+// it holds of the budget while it runs.
+uint64_t estimate(const sstg_graph *g, const sstg_request &r) {
+  switch (r.kind) {
+    case SSTG_REQ_BFS:
+      return g->n_rows * 4ull + bfs_bytes(g->n_rows);
+    case SSTG_REQ_CC:
+      return g->n_rows * 4ull + cc_bytes(g->n_rows);
+    default:
+      return least_bytes(g, r);
   }
 }
 
@@ -226,9 +242,11 @@ void reaper_main(sstg_server *S) {
     if (S->to_free.empty()) return;  // stopping with nothing left
     StoreSet t = S->to_free.back();
     S->to_free.pop_back();
+    S->reaping = true;
     lk.unlock();
     free_set_arrays(t);
     lk.lock();
+    S->reaping = false;
     S->reserved -= t.bytes;  // released only once actually freed
     S->cv.notify_all();
   }
@@ -608,7 +626,18 @@ void writer_main(sstg_server *S) {
 }
 
 bool admissible(sstg_server *S, const Request *q) {
-  if (S->reserved + q->est_bytes > S->budget) return false;
+  if (S->reserved + q->est_bytes > S->budget) {
+    if (S->running) return false;
+    // With no query running only store copies are in the way.  Spares make
+    // room (the reaper's wake-up brings the query here again); sets that
+    // waiting queries are pinned to go only once those have run.
+    for (const StoreSet &t : S->spare) S->to_free.push_back(t);
+    S->spare.clear();
+    if (S->reaping || !S->to_free.empty()) {
+      S->cv.notify_all();
+      return false;
+    }
+  }
   if (S->one_heavy && is_heavy(q->spec.kind) && S->heavy_running) return false;
   return free_slot(S) != nullptr;
 }
@@ -807,13 +836,14 @@ int sstg_server_submit(sstg_server *S, const sstg_request *req,
     r->src.assign(req->src, req->src + req->n);
     r->dst.assign(req->dst, req->dst + req->n);
   } else {
-    r->est_bytes = estimate(S->g, *req);
+    if (least_bytes(S->g, *req) > S->budget) {
+      delete r;
+      return SSTG_E_NOMEM;
+    }
+    // over the budget: the query gets all of it and runs alone
+    r->est_bytes = std::min(estimate(S->g, *req), S->budget);
   }
   std::lock_guard<std::mutex> lk(S->mu);
-  if (r->est_bytes > S->budget) {
-    delete r;
-    return SSTG_E_NOMEM;  // could never be admitted
-  }
   r->ticket = S->next_ticket++;
   S->all[r->ticket] = r;
   S->pending.push_back(r);

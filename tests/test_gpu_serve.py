@@ -205,3 +205,59 @@ def test_triangle_count_carried_through_updates():
         got, _, _ = _serve(n, s, d, reqs, slots=4, coalesce=True, snapshots=True,
                            one_heavy=one_heavy, maintain=True)
         _compare(reqs, got, exp)
+
+
+@pytest.mark.parametrize("kind,budget", [("bfs", 70), ("cc", 22)])
+def test_estimates_cover_the_scratch(kind, budget):
+    """A BFS takes up to 76 bytes a vertex on a graph of this size and a CC
+    24: under a budget (bytes a vertex) between the least a query is refused
+    by and those, queries run one at a time."""
+    need_gpu()
+    n, s, d = O.rmat_graph_edges(16, 8, 6)
+    g = S.SparseMatrixV(n)
+    g.insert_batch(s, d)
+    off, cols = g.export_csr()
+    hub = int(np.argmax(np.diff(off.astype(np.int64))))
+    want = O.bfs(off, cols, hub)[0] if kind == "bfs" else O.cc(off, cols)
+    srv = S.Server(g, slots=4, hbm_budget=n * budget, coalesce=True)
+    ts = [srv.bfs(hub) if kind == "bfs" else srv.cc() for _ in range(32)]
+    info = [srv.wait(t) for t in ts]
+    for t, i in zip(ts, info):
+        assert i["status"] == 0
+        assert np.array_equal(srv.fetch(t, np.uint32), want)
+    srv.close()
+    info.sort(key=lambda i: i["t_start"])
+    say(kind, "overlaps", sum(a["t_done"] > b["t_start"] for a, b in zip(info, info[1:])))
+    assert all(a["t_done"] <= b["t_start"] for a, b in zip(info, info[1:]))
+
+
+@pytest.mark.timeout(60)
+def test_spares_make_room_for_a_lone_query():
+    """A store copy kept for the next snapshot is given up when a query that
+    fits the budget only without it finds nothing else running: CCs (24 bytes
+    a vertex) leave room for a copy, a BFS (76) then does not fit beside it."""
+    need_gpu()
+    n, s, d = O.rmat_graph_edges(16, 8, 7)
+    g = S.SparseMatrixV(n)
+    g.insert_batch(s, d)
+    og = O.Graph(n)
+    og.insert_batch(s, d)
+    budget = n * 16 + 4 * g.statistics()["pool_capacity"] + 50 * n
+    srv = S.Server(g, slots=1, hbm_budget=budget, coalesce=False, snapshots=True)
+    rng = np.random.default_rng(9)
+    for i in range(4):
+        want = O.cc(*og.csr())
+        es, ed = rng.integers(0, n, (2, 200)).astype(np.uint32)
+        es, ed = np.concatenate([es, ed]), np.concatenate([ed, es])
+        checks = [(srv.cc(), want) for _ in range(8)]
+        srv.insert(es, ed)  # behind waiting queries: on a copy of the store
+        bfs = srv.bfs(i)
+        og.insert_batch(es, ed)
+        checks.append((bfs, O.bfs(*og.csr(), i)[0]))
+        for t, want in checks:
+            assert srv.wait(t)["status"] == 0
+            assert np.array_equal(srv.fetch(t, np.uint32), want)
+            srv.release(t)
+    say("store copies", srv.stats()["snapshots"])
+    assert srv.stats()["snapshots"] > 0
+    srv.close()
