@@ -3,8 +3,6 @@
 // kernel profiler, error notes).
 #include <cstdlib>
 
-#include <unordered_map>
-
 #include "algo.hpp"
 #include "graph.hpp"
 
@@ -97,113 +95,6 @@ void Profiler::reset() {
   flush();
   std::lock_guard<std::mutex> lk(mu);
   acc.clear();
-}
-
-// ------------------------------------------------------- device memory
-namespace {
-struct DevBlock {
-  void *p;
-  size_t bytes;
-  int dev;
-};
-// Never destroyed: graphs may be dropped while the process's statics go.
-struct DevCache {
-  std::mutex mu;
-  std::vector<DevBlock> idle;                   // newest last
-  std::unordered_map<void *, DevBlock> in_use;  // blocks dev_alloc handed out
-  size_t idle_bytes = 0;
-};
-DevCache &dev_cache() {
-  static DevCache *c = new DevCache();
-  return *c;
-}
-}  // namespace
-
-hipError_t dev_alloc(void **out, size_t bytes, size_t *got) {
-  DevCache &c = dev_cache();
-  *out = nullptr;
-  int dev = 0;
-  hipError_t e = hipGetDevice(&dev);
-  if (e != hipSuccess) return e;
-  if (!bytes) bytes = 1;
-  {
-    std::lock_guard<std::mutex> lk(c.mu);
-    size_t best = c.idle.size();
-    for (size_t i = 0; i < c.idle.size(); i++) {
-      const DevBlock &b = c.idle[i];
-      if (b.dev == dev && b.bytes >= bytes && b.bytes - bytes <= bytes / 2 &&
-          (best == c.idle.size() || b.bytes < c.idle[best].bytes))
-        best = i;
-    }
-    if (best < c.idle.size()) {
-      const DevBlock b = c.idle[best];
-      c.idle.erase(c.idle.begin() + (ptrdiff_t)best);
-      c.idle_bytes -= b.bytes;
-      c.in_use[b.p] = b;
-      *out = b.p;
-      if (got) *got = b.bytes;
-      return hipSuccess;
-    }
-  }
-  e = hipMalloc(out, bytes);
-  if (e == hipErrorOutOfMemory) {
-    (void)hipGetLastError();
-    dev_trim();
-    e = hipMalloc(out, bytes);
-  }
-  if (e != hipSuccess) {
-    *out = nullptr;
-    return e;
-  }
-  std::lock_guard<std::mutex> lk(c.mu);
-  c.in_use[*out] = DevBlock{*out, bytes, dev};
-  if (got) *got = bytes;
-  return hipSuccess;
-}
-
-void dev_free(void *p) {
-  if (!p) return;
-  DevCache &c = dev_cache();
-  std::vector<void *> back;
-  {
-    std::lock_guard<std::mutex> lk(c.mu);
-    auto it = c.in_use.find(p);
-    if (it == c.in_use.end() || it->second.bytes > kDevKeep / 2) {
-      if (it != c.in_use.end()) c.in_use.erase(it);
-      back.push_back(p);
-    } else {
-      c.idle.push_back(it->second);
-      c.idle_bytes += it->second.bytes;
-      c.in_use.erase(it);
-      while (c.idle_bytes > kDevKeep) {  // the oldest first
-        back.push_back(c.idle.front().p);
-        c.idle_bytes -= c.idle.front().bytes;
-        c.idle.erase(c.idle.begin());
-      }
-    }
-  }
-  for (void *q : back) (void)hipFree(q);
-}
-
-void dev_release(void *p) {
-  if (!p) return;
-  DevCache &c = dev_cache();
-  {
-    std::lock_guard<std::mutex> lk(c.mu);
-    c.in_use.erase(p);
-  }
-  (void)hipFree(p);
-}
-
-void dev_trim() {
-  DevCache &c = dev_cache();
-  std::vector<DevBlock> back;
-  {
-    std::lock_guard<std::mutex> lk(c.mu);
-    back.swap(c.idle);
-    c.idle_bytes = 0;
-  }
-  for (const DevBlock &b : back) (void)hipFree(b.p);
 }
 
 // ----------------------------------------------------------- workspace
@@ -744,8 +635,8 @@ int sstg_rmat(uint32_t n, uint32_t seed, double a, double b, double c,
     return SSTG_OK;
   }
   uint32_t *ds = nullptr, *dd = nullptr;
-  SSTG_HIP(hipMalloc(&ds, (count ? count : 1) * sizeof(uint32_t)));
-  SSTG_HIP(hipMalloc(&dd, (count ? count : 1) * sizeof(uint32_t)));
+  SSTG_HIP(dev_malloc(&ds, count * sizeof(uint32_t)));
+  SSTG_HIP(dev_malloc(&dd, count * sizeof(uint32_t)));
   int rc = rmat_generate(n, seed, a, b, c, first, count, ds, dd, s, norm);
   if (rc == SSTG_OK && count) {
     hipMemcpy(src, ds, count * sizeof(uint32_t), hipMemcpyDeviceToHost);
@@ -767,8 +658,8 @@ int sstg_er(uint32_t n, uint32_t seed, uint64_t first, uint64_t count,
     return SSTG_OK;
   }
   uint32_t *ds = nullptr, *dd = nullptr;
-  SSTG_HIP(hipMalloc(&ds, (count ? count : 1) * sizeof(uint32_t)));
-  SSTG_HIP(hipMalloc(&dd, (count ? count : 1) * sizeof(uint32_t)));
+  SSTG_HIP(dev_malloc(&ds, count * sizeof(uint32_t)));
+  SSTG_HIP(dev_malloc(&dd, count * sizeof(uint32_t)));
   int rc = er_generate(n, seed, first, count, ds, dd, nullptr);
   if (rc == SSTG_OK && count) {
     hipMemcpy(src, ds, count * sizeof(uint32_t), hipMemcpyDeviceToHost);
@@ -781,7 +672,7 @@ int sstg_er(uint32_t n, uint32_t seed, uint64_t first, uint64_t count,
 
 int sstg_device_alloc(uint64_t bytes, void **out) {
   if (!out) return SSTG_E_INVAL;
-  SSTG_HIP(hipMalloc(out, bytes ? bytes : 1));
+  SSTG_HIP(dev_malloc(out, bytes));
   return SSTG_OK;
 }
 

@@ -10,6 +10,7 @@
 #include <string>
 #include <vector>
 
+#include "device_memory.hpp"
 #include "sstg.h"
 
 namespace sstg {
@@ -73,30 +74,6 @@ Profiler &profiler();
                        __VA_ARGS__);                                          \
     if (p_.on) p_.end(#kernel, stream, ev_);                                  \
   } while (0)
-
-// ------------------------------------------------------- device memory
-// Device memory that outlives the graph it was allocated for: allocating and
-// freeing are the larger part of a short-lived graph's time (a hipFree waits
-// for the device and unmaps, 0.25 ms and more each; loading a rMat scale-20
-// graph and dropping it took 35 of them, 6.2 of 8.9 ms).  dev_free keeps a
-// block for the next dev_alloc of its device that it fits (at most half again
-// the size asked for), up to kDevKeep bytes in all; what is over goes back to
-// HIP, and everything does when an allocation fails and when the free memory
-// is asked for.  The caller of dev_free has waited for the work that used the
-// block: it may be handed to another stream at once.  dev_release gives a
-// block back to HIP in any case (waiting for the device, as hipFree does).
-// Any thread.  Blocks that dev_alloc did not make are passed on to hipFree.
-constexpr size_t kDevKeep = 4ull << 30;
-hipError_t dev_alloc(void **out, size_t bytes, size_t *got = nullptr);
-void dev_free(void *p);
-void dev_release(void *p);
-void dev_trim();
-template <class T> hipError_t dev_alloc(T **out, size_t bytes) {
-  void *p = nullptr;
-  const hipError_t e = dev_alloc(&p, bytes, nullptr);
-  *out = static_cast<T *>(p);
-  return e;
-}
 
 // ---------------------------------------------------------- workspace
 // Growable device scratch slots, reused across calls on one graph.  All use

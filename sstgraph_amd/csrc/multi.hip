@@ -454,20 +454,20 @@ int sstg_multi_create(uint32_t k, const uint32_t *n_per_graph,
     sstg_multi_destroy(M);
     return code;
   };
-  if (hipMalloc(&M->d_vbase, (k + 1) * sizeof(uint32_t)) ||
-      hipMalloc(&M->d_graph_of, n * sizeof(uint32_t)) ||
-      hipMalloc(&M->level, n * sizeof(uint32_t)) ||
-      hipMalloc(&M->label, n * sizeof(uint32_t)) ||
-      hipMalloc(&M->uf, n * sizeof(uint32_t)) ||
-      hipMalloc(&M->sources, k * sizeof(uint32_t)) ||
-      hipMalloc(&M->counts, kMultiCounts * sizeof(uint32_t)) ||
-      hipMalloc(&M->giant, k * sizeof(uint32_t)) ||
-      hipMalloc(&M->rank64, n * sizeof(double)) ||
-      hipMalloc(&M->c64a, n * sizeof(double)) ||
-      hipMalloc(&M->c64b, n * sizeof(double)) ||
-      hipMalloc(&M->rank32, n * sizeof(float)) ||
-      hipMalloc(&M->c32a, n * sizeof(float)) ||
-      hipMalloc(&M->c32b, n * sizeof(float)))
+  if (dev_malloc(&M->d_vbase, (k + 1) * sizeof(uint32_t)) ||
+      dev_malloc(&M->d_graph_of, n * sizeof(uint32_t)) ||
+      dev_malloc(&M->level, n * sizeof(uint32_t)) ||
+      dev_malloc(&M->label, n * sizeof(uint32_t)) ||
+      dev_malloc(&M->uf, n * sizeof(uint32_t)) ||
+      dev_malloc(&M->sources, k * sizeof(uint32_t)) ||
+      dev_malloc(&M->counts, kMultiCounts * sizeof(uint32_t)) ||
+      dev_malloc(&M->giant, k * sizeof(uint32_t)) ||
+      dev_malloc(&M->rank64, n * sizeof(double)) ||
+      dev_malloc(&M->c64a, n * sizeof(double)) ||
+      dev_malloc(&M->c64b, n * sizeof(double)) ||
+      dev_malloc(&M->rank32, n * sizeof(float)) ||
+      dev_malloc(&M->c32a, n * sizeof(float)) ||
+      dev_malloc(&M->c32b, n * sizeof(float)))
     return fail(SSTG_E_NOMEM);
   // on the stream the kernel below runs on (a copy on the null stream is
   // not ordered before work on it)

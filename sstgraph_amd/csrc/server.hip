@@ -210,7 +210,7 @@ int result_alloc(sstg_server *S, uint64_t bytes, void **out) {
       return SSTG_OK;
     }
   }
-  SSTG_HIP(hipMalloc(out, bytes));
+  SSTG_HIP(dev_malloc(out, bytes));
   return SSTG_OK;
 }
 
@@ -274,10 +274,10 @@ int detach_store(sstg_server *S) {
     S->reserved -= b.bytes;  // the spare becomes the graph's store
   } else {
     b.pool_cap = g->pool_cap;
-    if (hipMalloc(&b.off, (uint64_t)n * 8) != hipSuccess ||
-        hipMalloc(&b.deg, (uint64_t)n * 4) != hipSuccess ||
-        hipMalloc(&b.cap, (uint64_t)n * 4) != hipSuccess ||
-        hipMalloc(&b.pool, b.pool_cap * 4) != hipSuccess) {
+    if (dev_malloc(&b.off, (uint64_t)n * 8) != hipSuccess ||
+        dev_malloc(&b.deg, (uint64_t)n * 4) != hipSuccess ||
+        dev_malloc(&b.cap, (uint64_t)n * 4) != hipSuccess ||
+        dev_malloc(&b.pool, b.pool_cap * 4) != hipSuccess) {
       (void)hipGetLastError();
       free_set_arrays(b);
       return SSTG_E_NOMEM;
@@ -736,7 +736,7 @@ int view_init(sstg_graph *v, const sstg_graph *g) {
   v->device = g->device;
   SSTG_HIP(hipStreamCreateWithFlags(&v->stream, hipStreamNonBlocking));
   v->ws.stream = v->stream;
-  SSTG_HIP(hipMalloc(&v->dev_ctr, 16 * sizeof(uint64_t)));
+  SSTG_HIP(dev_malloc(&v->dev_ctr, 16 * sizeof(uint64_t)));
   SSTG_HIP(hipHostMalloc(&v->host_rb, 64 * sizeof(uint64_t),
                          hipHostMallocDefault));
   v->version = ~0ull;

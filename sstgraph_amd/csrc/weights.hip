@@ -262,8 +262,8 @@ int wt_reserve(sstg_graph *g, uint64_t extra) {
   uint64_t cap = 1024;
   while (cap < 4 * (g->wt_live + extra)) cap <<= 1;
   unsigned long long *keys = nullptr, *vals = nullptr;
-  SSTG_HIP(hipMalloc(&keys, cap * 8));
-  if (hipMalloc(&vals, cap * 8) != hipSuccess) {
+  SSTG_HIP(dev_malloc(&keys, cap * 8));
+  if (dev_malloc(&vals, cap * 8) != hipSuccess) {
     (void)hipGetLastError();
     hipFree(keys);
     return SSTG_E_NOMEM;
