@@ -1,13 +1,13 @@
 """The symmetry check: edges without a reverse that point up, down or both in
 the (degree, id) order, with edge counts around a block's 2048.  A graph taken
-for symmetric by mistake shows in BFS, whose bottom-up steps follow rows the
-wrong way."""
+for symmetric by mistake shows in BC, which then sums a vertex's paths over
+its own row: 0 for a vertex reached by such an edge alone."""
 import numpy as np
 import pytest
 
 import sstgraph_amd as S
 from oracle import oracle as O
-from tests.gpu_common import need_gpu, say
+from tests.gpu_common import need_gpu, rel_close, say
 
 pytestmark = pytest.mark.gpu
 
@@ -35,8 +35,11 @@ def test_edges_without_reverse(lone, pairs):
     g = S.SparseMatrixV(n)
     g.insert_batch(s, d)
     for src in (hub, int(s[0]), n - 1):
-        say("bfs", lone, pairs, len(cols), src)
+        say("bfs, bc", lone, pairs, len(cols), src)
         want, _ = O.bfs(off, cols, src)
         parent, level = S.EdgeMapVertexMap.BFS(g, src, levels=True)
         assert np.array_equal(level, want)
         assert np.array_equal(parent >= 0, want != S.UNREACHED)
+        got = S.EdgeMapVertexMap.BC(g, src)
+        ok, worst = rel_close(got, O.bc(off, cols, src), 1e-9, 1e-12)
+        assert ok, worst

@@ -5,13 +5,13 @@ handles: in-place and relocated rows, hub rows moved by the whole
 workgroup, removes of many ids of one row, duplicates and self-loops, and
 the cases it hands back to the general pipeline (no pool room, a row
 moving more than 2^15 ids).  Symmetry tracked through small batches keeps
-BFS bottom-up steps exact."""
+BFS, and BC's sums over a vertex's own row, exact."""
 import numpy as np
 import pytest
 
 import sstgraph_amd as S
 from oracle import oracle as O
-from tests.gpu_common import assert_same_csr, need_gpu, say
+from tests.gpu_common import assert_same_csr, need_gpu, rel_close, say
 
 pytestmark = pytest.mark.gpu
 EMV = S.EdgeMapVertexMap
@@ -132,4 +132,6 @@ def test_small_symmetric_batches_keep_bfs_exact():
         src = int(np.argmax(np.diff(off)))
         _, lev = EMV.BFS(g, src, levels=True)
         assert np.array_equal(lev, O.bfs(off, cols, src)[0]), step
+        ok, worst = rel_close(EMV.BC(g, src), O.bc(off, cols, src), 1e-9, 1e-12)
+        assert ok, (step, worst)
     assert_same_csr(g, og, "end")
