@@ -126,3 +126,60 @@ def test_directed_frontier_of_sinks(sinks, edges):
     assert np.array_equal(EMV.BF(g, src), O.bf(off, cols, src))
     ok, worst = rel_close(EMV.BC(g, src), O.bc(off, cols, src), 1e-9, 1e-12)
     assert ok, worst
+
+
+def _layers(flip, rng):
+    """A source, 2^16 vertices behind it, and two more layers with degrees on
+    both sides of every pull class (32, 128, 2048), the last with neighbours
+    in the middle one only; flip: ids reversed, so rows are read from the
+    other end."""
+    near = np.arange(1, (1 << 16) + 1)
+    per = {1: 20000, 8: 20000, 32: 3000, 33: 3000, 128: 600, 129: 600,
+           2048: 100, 2049: 100, 6000: 30}
+    degree = np.repeat(list(per), list(per.values()))
+    mid = near[-1] + 1 + np.arange(len(degree))
+    far = mid[-1] + 1 + np.arange(len(degree) // 10)
+    ends = [(np.zeros(len(near), int), near)]
+    for ids, back, deg in ((mid, near, degree), (far, mid, degree[::10])):
+        s = np.repeat(ids, deg)
+        ends.append((s, rng.choice(back, len(s))))
+    s = np.concatenate([x for x, _ in ends])
+    d = np.concatenate([y for _, y in ends])
+    s, d = np.concatenate([s, near]), np.concatenate([d, rng.permutation(near)])
+    extra = rng.choice(near, (2, 1200000))  # over 2^22 edges in all
+    s, d = np.concatenate([s, extra[0]]), np.concatenate([d, extra[1]])
+    n = int(far[-1]) + 2  # and one vertex of no edge
+    return (n, n - 1 - s, n - 1 - d, n - 1) if flip else (n, s, d, 0)
+
+
+@pytest.mark.parametrize("flip", [False, True])
+def test_bottom_up_steps(flip):
+    """A graph too large to stay on the device whose second and third steps
+    are bottom-up, with vertices of every pull class found in each."""
+    need_gpu()
+    n, s, d, src = _layers(flip, np.random.default_rng(11))
+    off, cols, g = _check(n, s, d, [src])
+    assert len(cols) > 1 << 22
+    alpha, beta = g.bfs_switch()
+    level, _ = O.bfs(off, cols, src)
+    deg = np.diff(off).astype(np.int64)
+    size = [(level == k).sum() for k in range(4)]
+    edges = [deg[level == k].sum() for k in range(4)]
+    # the second step: over the cap, growing, and over the rest's share
+    assert edges[1] > CAP and size[1] > size[0]
+    assert edges[1] > (len(cols) - edges[0] - edges[1]) / alpha
+    assert size[2] >= n / beta  # the third stays bottom-up
+    for k in (2, 3):
+        assert (np.histogram(deg[level == k], [1, 33, 129, 2049, 1 << 32])[0] > 0).all()
+
+
+@pytest.mark.parametrize("flip", [False, True])
+def test_one_edge_without_reverse(flip):
+    """The same graph with one edge more, the only one of the vertex it ends
+    at: bottom-up steps would miss that vertex."""
+    need_gpu()
+    n, s, d, src = _layers(flip, np.random.default_rng(11))
+    lone, near = (0, n - 2 - 77) if flip else (n - 1, 1 + 77)
+    s, d = np.concatenate([s, d, [near]]), np.concatenate([d, s, [lone]])
+    off, cols, _ = _check(n, s, d, [src], False)
+    assert O.bfs(off, cols, src)[0][lone] == 2
