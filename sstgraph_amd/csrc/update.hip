@@ -639,11 +639,15 @@ __global__ void __launch_bounds__(kT)
 // the 1e7-edge batch).  Each lane first walks the chain of descriptors of one
 // row (segment, vertex, slot), so a wave pays those round trips once.
 //
-// Bound by the latency of its loads (waves wait three quarters of their
-// cycles; 2.5 GB of traffic at 3.8 TB/s).  1e7-edge insert at rMat scale 24, 3.34M rows,
-// 220M outputs: 0.66 ms, where inputs staged in LDS and ranked by binary
-// searches among the other side's values took 0.87 and 0.09 for descriptors
-// and degrees; a wave per row with the keys as scalars took 1.0-1.6.
+// Few rows have a wave each: 64 rows of 1,550 inputs four to a wave made a
+// 1e5-edge insert 177 us, one to a wave 145; with 16,384 rows so the same insert
+// went from 143 to 150, and with 9,300 from 118 to 124.
+//
+// Bound by bytes: the 1e7-edge insert at rMat scale 24 (3.34M rows, 220M
+// outputs) moves 2.78 GB in 0.64-0.69 ms, 4.0-4.3 TB/s where a large copy
+// reaches 4.94.  Inputs staged in LDS and ranked by binary searches among the
+// other side's values took 0.87 ms and 0.09 for descriptors and degrees; a
+// wave per row with the keys as scalars 1.0-1.6.
 constexpr int kRowT = 256;
 constexpr int kRowWaves = kRowT / kWave;
 constexpr uint32_t kRowWindow = 4096;    // flat positions at a time
@@ -651,6 +655,7 @@ constexpr int kRowsAhead = 4;            // pieces of 64 per group of loads
 constexpr uint32_t kRowLane = 8;         // keys up to which a lane sets its row's
 constexpr uint64_t kRowSpread = 16384;   // waves wanted
 constexpr uint32_t kRowRun = 4;          // consecutive rows of a wave
+constexpr uint64_t kRowAlone = 4096;     // rows up to which each has a wave
 static_assert(kTileMax <= (int)kRowWindow, "a row fits a window");
 static_assert(kRowWindow == 64 * kWave, "a lane per 64 positions");
 
@@ -665,8 +670,9 @@ __global__ void __launch_bounds__(kRowT)
   const uint32_t *blo = reinterpret_cast<const uint32_t *>(a.B);
   const uint64_t wave = (uint64_t)blockIdx.x * kRowWaves + w;
   const uint64_t waves = (uint64_t)gridDim.x * kRowWaves;
+  const uint32_t run = per < kRowRun ? 1u : kRowRun;
   const uint64_t mine =
-      ((uint64_t)(lane / kRowRun) * waves + wave) * kRowRun + lane % kRowRun;
+      ((uint64_t)(lane / run) * waves + wave) * run + lane % run;
   const bool have = lane < per && mine < a.nt;  // a prefix of the lanes
   const uint32_t nrows = (uint32_t)__popcll(__ballot(have));
   if (nrows == 0) return;  // whole waves (no block barrier below)
@@ -1281,8 +1287,11 @@ static int update_chunk(sstg_graph *g, const uint32_t *src, const uint32_t *dst,
   if (nt) {
     // enough waves to fill the chip, and up to 64 rows each
     const uint64_t want = ceil_div(nt, kRowSpread);
-    const uint32_t per = (uint32_t)(
-        want >= kWave ? kWave : ceil_div(want, kRowRun) * kRowRun);
+    const uint32_t per =
+        nt <= kRowAlone ? 1u
+                        : (uint32_t)(want >= kWave
+                                         ? kWave
+                                         : ceil_div(want, kRowRun) * kRowRun);
     const uint64_t nblk = ceil_div(ceil_div(nt, (uint64_t)per), kRowWaves);
     if (insert)
       SSTG_LAUNCH(k_merge_rows<true>, nblk, kRowT, 0, s, a,

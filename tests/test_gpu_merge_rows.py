@@ -43,6 +43,18 @@ def _batch(lengths, keys, where, rng):
     [4095, 4096, 2048, 63, 64, 65, 1, 1400, 1400] * 80,
 ], ids=["empty", "short", "longest", "mixed"])
 def test_rows(lengths, keys, where):
+    _check(lengths, keys, where)
+
+
+@pytest.mark.parametrize("rows,length,keys", [
+    (3, 1000, 1450), (5, 0, 1530), (64, 900, 600), (4095, 60, 3),
+    (4096, 700, 2), (4097, 700, 2), (4099, 30, 70), (16385, 100, 2)])
+def test_row_counts(rows, length, keys):
+    """Up to 4096 rows have a wave each, more share waves four at a time."""
+    _check([length] * rows, keys, "any")
+
+
+def _check(lengths, keys, where):
     need_gpu()
     rng = np.random.default_rng([keys, len(lengths)])
     g, og = S.SparseMatrixV(N), O.Graph(N)
