@@ -94,9 +94,23 @@ constexpr uint32_t kPushTile = kPushT * kPushPer;  // most edges per tile
 constexpr uint32_t kPushGrid = 256;
 constexpr int kPushCountBits = 24;
 constexpr uint64_t kPushCountMask = (1ull << kPushCountBits) - 1;
-constexpr int kPushLevels = 12;  // most levels per batch
-// a frontier of more edges goes back to the host, which may turn bottom-up or
-// launch a push sized to it; a graph of at most kPushAll edges stays here
+// Most levels per batch, a third of them in a graph of over kPushAll edges,
+// whose middle levels go back to the host: too few cost read-backs, too many
+// launches that find nothing to do.  BFS from the hub in us with 6 / 12 / 24:
+// rMat scale 16 149 / 138 / 158, scale 17 186 / 169 / 190; with a third of
+// 2 / 4 / 8: 8.4M Erdos-Renyi edges 195 / 176 / 200, rMat scale 20
+// 354 / 348 / 370 (a 2000 x 2000 grid of 4,000 levels 63 / 52 / 47 ms).  A
+// BFS of one or two levels pays for the rest: from a star's centre 106 us,
+// 84 with a read-back per level.
+constexpr int kPushLevels = 12;
+// A frontier of more edges goes back to the host, which may turn bottom-up or
+// launch a push sized to it; a graph of at most kPushAll edges stays here.
+// kPushCap from 2^18 to 2^22: rMat scale 22 585 593 583 572 590 us, scale 24
+// 1201 1169 1169 1156 1128, 67M Erdos-Renyi edges 552 549 545 541 570.
+// kPushAll from 2^20 to 2^24: rMat scale 17 (2.4M edges) 208 209 170 166 170
+// us, Erdos-Renyi of 4.2M 129 140 154 153 149, of 8.4M 163 172 176 213 211,
+// rMat scale 19 (10M) 270 269 282 285 338, Erdos-Renyi of 17M 213 213 215 214
+// 425: a graph kept here does without the bottom-up steps.
 constexpr uint64_t kPushCap = 1ull << 20;
 constexpr uint64_t kPushAll = 1ull << 22;
 
@@ -651,8 +665,9 @@ __global__ void k_sigma_push(DevGraph g, const uint32_t *list, uint64_t count,
 // many, every edge has one.  So only the first kind is searched, half of the
 // edges and each in the shorter of the two rows.  Clears *flag at an edge
 // without its reverse; part gets each block's difference of the two kinds.
-// Searching every edge in its other end's row took the first BFS
-// of a rMat scale-24 graph from 15.7 to 33.0 ms, 10.1 at scale 22 against 5.4.
+// The first BFS of a rMat scale-24 graph, which checks it, takes 15.7 ms, and
+// BC at scale 22 5.4; with every edge searched in its other end's row they
+// took 33.0 and 10.1.
 __global__ void __launch_bounds__(kT)
     k_symmetry(DevGraph g, const uint64_t *prefix, uint64_t m, uint32_t *flag,
                int64_t *part) {
@@ -789,6 +804,9 @@ struct BfsRun {
 // frontier found, [5] size of the frontier before the current one, [6]
 // degree sum of the current frontier; ends[k] = end of the frontier found by
 // the k-th level run.
+// Bounds: one block is slow over levels that the device-driven batches spread
+// over the chip (a 2000 x 2000 grid 48 / 51 / 84 ms with up to 1024 / 4096 /
+// 16384 edges, rMat and Erdos-Renyi graphs the same within 2%).
 constexpr uint32_t kTailThreads = 1024;
 constexpr uint32_t kTailFrontier = 4096;
 constexpr uint32_t kTailEdges = 4096;
@@ -1341,7 +1359,7 @@ int algo_cc(sstg_graph *g, uint32_t *out) {
   const DevGraph v = g->view();
   if (g->m && symmetric) {
     uint32_t *samples = nullptr;
-    // PageRank's contribution buffer holds the same bytes (8 per vertex)
+    // FP64 PageRank's contribution buffer has the same bytes (8 per vertex)
     SSTG_TRY(g->ws.get(kWsAlgo + 20, (uint64_t)n * cc::kHookRounds, &samples));
     const cc::Slots sl{prefix, nullptr, nullptr, n};
     SSTG_TRY(cc::forest_symmetric(v, sl, p, samples, 1, giant, s));

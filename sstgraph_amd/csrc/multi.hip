@@ -297,7 +297,9 @@ static int capture(sstg_multi *M, uint32_t max_levels, uint32_t iters,
   bool symmetric = false;
   SSTG_TRY(graph_is_symmetric(g, &symmetric));
   uint32_t *samples = nullptr;
-  // PageRank's contribution buffer holds the same bytes (8 per vertex)
+  // a slot of the union store's own, 8 bytes a vertex (the batched PageRank
+  // has buffers apart); only PageRank and CC called on the union store itself
+  // share it, with no more bytes, so the recorded address stays
   SSTG_TRY(g->ws.get(kWsAlgo + 20, (uint64_t)n * cc::kHookRounds, &samples));
   SSTG_HIP(hipStreamSynchronize(s));
   // the event profiler must not record into a capturing stream
