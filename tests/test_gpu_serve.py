@@ -209,7 +209,7 @@ def test_triangle_count_carried_through_updates():
 
 @pytest.mark.parametrize("kind,budget", [("bfs", 70), ("cc", 22)])
 def test_estimates_cover_the_scratch(kind, budget):
-    """A BFS takes up to 76 bytes a vertex on a graph of this size and a CC
+    """A BFS takes up to 84 bytes a vertex on a graph of this size and a CC
     24: under a budget (bytes a vertex) between the least a query is refused
     by and those, queries run one at a time."""
     need_gpu()
@@ -235,7 +235,7 @@ def test_estimates_cover_the_scratch(kind, budget):
 def test_spares_make_room_for_a_lone_query():
     """A store copy kept for the next snapshot is given up when a query that
     fits the budget only without it finds nothing else running: CCs (24 bytes
-    a vertex) leave room for a copy, a BFS (76) then does not fit beside it."""
+    a vertex) leave room for a copy, a BFS (84) then does not fit beside it."""
     need_gpu()
     n, s, d = O.rmat_graph_edges(16, 8, 7)
     g = S.SparseMatrixV(n)
